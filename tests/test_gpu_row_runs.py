@@ -1,0 +1,59 @@
+"""The expert-major decode products where an expert has as many rows as a pass takes, one fewer, one
+more, several passes' worth, or more runs than there are workgroup columns for - and uneven K
+quarters - against the oracle's layer. A router bias sends every token to the same experts, so their
+row counts are the token count exactly."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+from gpu_helpers import announce, assert_bf16_bar, bf16_bits, bf16_values, normal_bf16
+from test_gpu_layer_routing import quantised
+from uniserve_moe import ops
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    # name: tokens, hidden, experts, top, intermediate, window, live
+    "a pass less one": (31, 512, 64, 4, 256, None, None),
+    "a pass": (32, 1024, 64, 4, 256, None, None),
+    "a pass and one": (33, 512, 64, 4, 256, None, None),
+    "two passes and one, 20 and 6 lines of K": (65, 1280, 64, 4, 384, None, None),
+    "some rows not live": (100, 512, 64, 4, 256, None, 70),
+    "fewer columns than passes": (300, 512, 128, 8, 256, (2, 3), None),
+    "fewer columns than passes, a run ends on a pass": (288, 512, 128, 8, 256, (0, 4), None),
+    "fewer routes than experts": (40, 512, 128, 2, 256, None, None),
+}
+
+
+@pytest.mark.parametrize("wdtype", ["bf16", "f8e4m3", "f4e2m1"])
+@pytest.mark.parametrize("case", list(CASES))
+def test_experts_of_many_rows(device, case, wdtype):
+    tokens, hidden, experts, top, intermediate, window, live = CASES[case]
+    if wdtype == "f4e2m1":
+        intermediate = 512 if intermediate == 384 else intermediate  # whole 256-element chunks
+    announce("row runs", case, wdtype)
+    offset, local = (0, experts) if window is None else window
+    x = normal_bf16((tokens, hidden), 81, device=device)
+    router = normal_bf16((experts, hidden), 82, 0.02, device)
+    up_gate = normal_bf16((local, 2 * intermediate, hidden), 83, 0.02, device)
+    down = normal_bf16((local, hidden, intermediate), 84, 0.02, device)
+    bias = np.where(np.arange(experts) < top, 40.0, 0.0).astype(np.float32)
+    w1, w2, s1, s2, up_dev, down_dev, args = quantised(wdtype, up_gate, down, device)
+    layer = ops.MoeLayer(hidden, experts, top, intermediate, tokens, weight_dtype=wdtype)
+    live_t = None if live is None else torch.tensor([live], dtype=torch.int32, device=device)
+    out = layer(x, router, up_dev, down_dev, router_bias=torch.from_numpy(bias).to(device), live_tokens=live_t,
+                window=window, **args)
+    torch.cuda.synchronize()
+    got = bf16_values(out)
+    want_bits, want_ids, _, _ = O.moe_layer(
+        bf16_bits(x), bf16_bits(router), w1, w2, top, up_gate_scales=s1, down_scales=s2, router_bias=bias, live=live,
+        window=None if window is None else (offset, local))
+    ids = layer.view("ids", torch.int32, (tokens, top)).cpu().numpy()
+    served = tokens if live is None else live
+    np.testing.assert_array_equal(ids[:served], want_ids[:served])
+    assert (np.sort(ids[:served], axis=1) == np.arange(top)).all()  # every token names the same experts
+    assert (got[served:] == 0).all()
+    assert_bf16_bar(got[:served], O.bf16_decode(want_bits).astype(np.float64)[:served], case,
+                    max_rel=2e-2 if wdtype == "bf16" else 4e-2)

@@ -121,6 +121,21 @@ __device__ __forceinline__ void store_device(T *pointer, T value) {
   __hip_atomic_store(pointer, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ---- buffer loads -------------------------------------------------------------------------------------
+
+/// A uniform base address whose loads take one 32-bit lane offset and one uniform offset each, both
+/// below 4 GiB: no address arithmetic and no 64-bit address registers per load.
+typedef __amdgpu_buffer_rsrc_t BufferBase;
+__device__ __forceinline__ BufferBase buffer_base(const void *pointer, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(pointer), 0, bytes, 0x00027000);
+}
+/// 16 bytes at base + lane_offset + offset (kOnce: non-temporal).
+template <bool kOnce>
+__device__ __forceinline__ uint32_t __attribute__((ext_vector_type(4)))
+buffer_load16(BufferBase base, uint32_t lane_offset, uint32_t offset) {
+  return __builtin_amdgcn_raw_buffer_load_b128(base, lane_offset, offset, kOnce ? 2 : 0);
+}
+
 // ---- MFMA operands ------------------------------------------------------------------------------------
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

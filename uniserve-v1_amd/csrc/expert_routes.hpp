@@ -112,6 +112,78 @@ __device__ __forceinline__ int32_t nth_named_expert(const int32_t *ids, int64_t 
   return -1;
 }
 
+/// A run of an expert's listed rows.
+struct RowRun {
+  int32_t expert;  ///< local expert, or -1: no such run
+  int32_t first;   ///< its first row
+  int32_t rows;    ///< rows it covers (the expert's last run: fewer may be left)
+};
+
+/// The n-th of at most `columns` runs (columns >= the smaller of local_experts and
+/// (routes - 1) / kRows) covering every row past the experts' first kRows each, experts ascending,
+/// rows ascending: runs of kRows rows, or of the smallest doubling of it with which `columns` runs
+/// are enough. The workgroup counts every local expert's live routes in `counts` (LDS,
+/// local_experts words) and scans the experts' run counts. Every thread of the workgroup calls it
+/// and gets the same answer; `counts` is free again when it returns.
+template <int kThreads, int kRows>
+__device__ __forceinline__ RowRun nth_extra_run(const int32_t *ids, int64_t routes, int64_t live, int32_t local_offset,
+                                                int32_t local_experts, int n, int columns, int32_t *counts) {
+  constexpr int kWaves = kThreads / kWave;
+  __shared__ int32_t wave_runs[2][kWaves];
+  __shared__ RowRun found;
+  const int t = static_cast<int>(threadIdx.x);
+  for (int e = t; e < local_experts; e += kThreads) counts[e] = 0;
+  if (t == 0) found = RowRun{-1, 0, 0};
+  __syncthreads();
+  const int64_t last = routes < live ? routes : live;
+  constexpr int kAhead = 8;  // ids in flight per thread
+  for (int64_t at = t; at < last; at += kAhead * kThreads) {
+    int32_t local[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int64_t route = at + u * kThreads;
+      local[u] = route < last ? ids[route] - local_offset : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (local[u] >= 0 && local[u] < local_experts) atomicAdd(counts + local[u], 1);
+  }
+  __syncthreads();
+  // Thread t's experts: [t each, (t + 1) each).
+  const int each = (local_experts + kThreads - 1) / kThreads;
+  auto runs_of = [&](int e, int rows) { return e < local_experts && counts[e] > kRows ? (counts[e] - kRows + rows - 1) / rows : 0; };
+  int rows = kRows, own, upto, parity = 0;
+  for (;; rows *= 2, parity ^= 1) {
+    own = 0;
+    for (int i = 0; i < each; ++i) own += runs_of(t * each + i, rows);
+    upto = own;  // inclusive scan over the wavefront
+#pragma unroll
+    for (int step = 1; step < kWave; step *= 2) {
+      const int before = __shfl_up(upto, step, kWave);
+      if (lane_id() >= step) upto += before;
+    }
+    if (lane_id() == kWave - 1) wave_runs[parity][t / kWave] = upto;
+    __syncthreads();
+    int total = 0;
+    for (int w = 0; w < kWaves; ++w) total += wave_runs[parity][w];
+    if (total <= columns || rows >= static_cast<int>(routes)) break;  // (uniform; one run per expert at most)
+  }
+  int at = upto - own;
+  for (int w = 0; w < t / kWave; ++w) at += wave_runs[parity][w];
+  if (n >= at && n < at + own) {
+    for (int i = 0; i < each; ++i) {
+      const int runs = runs_of(t * each + i, rows);
+      if (n < at + runs) {
+        found = RowRun{t * each + i, kRows + (n - at) * rows, rows};
+        break;
+      }
+      at += runs;
+    }
+  }
+  __syncthreads();
+  return found;
+}
+
 /// Row m of the list (m < the total).
 template <int kWaves>
 __device__ __forceinline__ int64_t listed_route(const int32_t *list, const int32_t *counts, int64_t routes, int m) {

@@ -20,14 +20,15 @@ struct ExpertStream {
   const int32_t *ids;        ///< [routes] expert ids after the slot map
   const int32_t *live_tokens;///< [1] or null
   int64_t routes, top, local_offset, local_experts;
+  int64_t experts;           ///< the router's (routes / experts: the rows an expert expects)
   int64_t K, n_total, out_width;
   int32_t activation;        ///< FC1's gate
 };
 
 /// Whether the expert-major stream kernels serve these extents (decode batches: at most 4096
-/// routes, fewer than 24 per local expert - with fewer routes than local experts a compact grid over
+/// routes, fewer than 24 per expert on average - with fewer routes than local experts a compact grid over
 /// at most 512 of them; FC1 widths of whole 64-column slices, FC2 of whole 128-column ones).
-bool expert_stream_fits(int64_t routes, int64_t local_experts, int64_t K, int64_t out_width, bool gated);
+bool expert_stream_fits(int64_t routes, int64_t experts, int64_t local_experts, int64_t K, int64_t out_width, bool gated);
 
 /// FC1 (`gated`: the gate of `activation` times the up half) or FC2 over the listed routes.
 void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream);

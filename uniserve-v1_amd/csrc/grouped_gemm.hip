@@ -11,17 +11,19 @@
 // accumulation, the activation on the accumulators, one rounding into bf16; rows past a tile's
 // limit are neither read nor stored.
 //
-// Three kernels per product, chosen on the host from the expected rows per expert (tokens x top /
+// The kernels of each product, chosen on the host from the expected rows per expert (tokens x top /
 // experts), which is all the host knows without reading device memory, and from the shape:
 //
-//  * `stream` (decode: a few rows per expert). Weight-streaming bound: every touched expert's
-//    matrix is read once from HBM and nothing else matters. A workgroup owns one tile and a
-//    128-row slice of the expert's weight rows; each wavefront streams its 32 weight rows as whole
-//    non-temporal 128-byte lines into registers and regroups them into the MFMA operand layout
-//    through its own LDS buffer, the tile's activation rows coming from L2. The weight rows are MFMA
-//    operand A and the activation rows operand B (16x16x32 bf16), so each lane ends holding four
-//    consecutive output columns of one row - an 8-byte store - and the SiLU pair (up column n,
-//    gate column n) meets in one lane. Tiles of more than 32 rows are covered in passes of 32.
+//  * `wide` (decode and continuous batches: up to two dozen rows per expert). Weight-streaming bound:
+//    every touched expert's matrix is read from HBM and little else matters. A workgroup owns 128
+//    weight rows and 32 activation rows, its wavefronts a quarter of K each.
+//
+//  * `stream` (FC2 of the smallest batches, and K below 256): a 128-row slice of the expert's weight
+//    rows per workgroup, each wavefront streaming its own 32 rows over all of K. The weight lines are
+//    regrouped into the MFMA operand layout through LDS, the activation rows come from L2. The weight
+//    rows are MFMA operand A and the activation rows operand B (16x16x32 bf16), so each lane ends
+//    holding four consecutive output columns of one row - an 8-byte store - and the SiLU pair (up
+//    column n, gate column n) meets in one lane.
 //
 //  * `prefill` (grouped_prefill.hpp; hundreds of rows per expert): 128 x 512 tiles of 8
 //    wavefronts, both operands DMA'd into LDS, for the shapes it serves.
@@ -67,6 +69,8 @@ struct GroupedParams {
   int64_t routes;
   int64_t local_offset;
   int64_t local_experts;
+  int32_t columns;          ///< wide kernel, expert-major: workgroup columns (experts, or routes if compact)
+  int32_t extra_columns;    ///< wide kernel: workgroup columns past the experts', for rows past an expert's first pass
   int32_t compact;          ///< workgroup x serves the x-th named local expert (fewer routes than experts)
 };
 
@@ -83,12 +87,6 @@ __device__ __forceinline__ void store_bf16x4(uint16_t *pointer, floatx4 v) {
 
 // ---- stream kernel (decode) ----------------------------------------------------------------------------
 
-/// Average routes per expert at or below which the stream kernel takes a tile in passes of one
-/// 16-row MFMA block instead of two (at 64-token decode: FC2 63.7 against 66.2 us with two, FC1
-/// 124 against 125); a tile with more rows re-streams its weights per pass, which at such
-/// averages is rare.
-constexpr int64_t kOnePassRowsPerExpert = 8;
-
 //
 // Grid: (max tiles, weight-row slices). FC1 slices are 64 gated columns (64 up + 64 gate rows),
 // FC2 slices 128 output columns; wavefront w takes 16 + 16 of them. Needs K % 128 == 0.
@@ -104,14 +102,14 @@ constexpr int64_t kOnePassRowsPerExpert = 8;
 // K mapping (the same for weights and activations): step s in 0..3 of a stage, lane group
 // g = l / 16 takes the stage's 16-byte chunk 4 s + g, i.e. line s / 2, chunk 4 (s % 2) + g.
 
-/// kPassTiles: rows of a tile one pass covers, in MFMA blocks of 16.
 /// kByExpert: workgroup x serves local expert x (grid: local experts x slices) and finds its rows
 /// itself - the routes whose id is the expert's, in route order, live ones only (each wavefront
 /// ballots a quarter of the routes into a list in LDS) - while its first weight stage is in
 /// flight; FC1 reads token route / top and FC2 row `route`, and both write row `route` (the
 /// expanded layout). Otherwise the sort's tile tables give the tile's expert and rows.
-template <bool kGated, int kPassTiles, bool kByExpert = false>
+template <bool kGated, bool kByExpert>
 __global__ void __launch_bounds__(kThreads) stream_kernel(GroupedParams p) {
+  constexpr int kPassTiles = 1;  // 16-row MFMA blocks per pass
   const int wave = static_cast<int>(threadIdx.x) / kWave;
   const int lane = lane_id();
   const int r16 = lane & 15;
@@ -283,141 +281,236 @@ __global__ void __launch_bounds__(kThreads) stream_kernel(GroupedParams p) {
   }
 }
 
-// ---- quarter kernel (decode, expert-major) ----------------------------------------------------------------
+// ---- wide kernel (decode and continuous batches) -----------------------------------------------------------
 //
-// FC1's gated product with the workgroup's 128 weight rows (64 up + the matching 64 gate rows)
-// streamed by every wavefront over its own quarter of K: wavefront q walks K
-// lines q K / 256 .. (q + 1) K / 256 - 1 (64 bf16 each) of all 128 rows, one step = one line of 64
-// rows (8 instructions of 8 rows x 128 bytes), the two halves of the rows in turn. At any moment
-// the workgroup's four wavefronts read four neighbouring stretches of the same rows, which DRAM
-// serves from fewer row openings than the row-sliced walk, where each wavefront reads 256 bytes of
-// its own rows per stage (a bare kernel reading FC1's weights: 7.2 against 6.3 TB/s). Each
-// wavefront holds partial sums of all 128 rows; at the end they meet in LDS and wavefront w adds
-// the four in wave order for its output rows (up set w and gate set w + 4: 16 gated columns).
-// FC1 from 124 to 120 us at 30B T=64; FC2 (128 rows of one kind) measured 1 us slower, so it keeps
-// the row-sliced kernel. Needs K % 256 == 0 and byte offsets of an expert's weights and of the
+// A workgroup owns 128 weight rows (FC1: 64 up + the matching 64 gate rows; FC2: 128 output columns)
+// and takes 32 activation rows per pass; wavefront q streams all 128 rows over its own quarter of K
+// (L = K / 64 lines of 64 bf16: lines q L / 4 .. (q + 1) L / 4 - 1), one step = one line of 64 rows
+// (8 instructions of 8 rows x 128 bytes), the two halves of the rows in turn. At any moment the
+// workgroup's four wavefronts read neighbouring stretches of the same rows, which DRAM serves from
+// fewer row openings than the row-sliced walk, where each wavefront reads 256 bytes of its own rows
+// per stage (a bare kernel reading FC1's weights: 7.2 against 6.3 TB/s), and each activation byte is
+// loaded by one wavefront of the workgroup instead of by all four (loads in the operand layout go at
+// about 16 B/clk per CU, so four times the rows' bytes were the row-sliced kernel's bound from about
+// eight rows per expert). The partial sums meet in LDS, added in wave order.
+//
+// Bound by HBM: 30B (H 2048, I 768, 128 experts) T=64 FC1 117 us, 6.9 TB/s. Against 16 rows a pass
+// (the weights streamed again for each 16 rows) and FC2 row-sliced: T=128 FC1 132 -> 122 us, FC2 70
+// -> 65; T=200 166 -> 124, 73 -> 70; T=301 220 -> 138, 92 -> 83. A third block of 16 rows spills
+// (T=301 FC1 166).
+//
+// Expert-major (kByExpert): an expert's first workgroups take its first 32 rows; the workgroups
+// dispatched last share out the rows past those (nth_extra_run), so a much-named expert's passes run
+// side by side: 30B T=301 with Zipf(1.1) routing FC1 314 -> 142 us, FC2 181 -> 92. They come last
+// since most find nothing to do, and at the kernel's end the slots they hold are idle anyway (first:
+// T=200 near-uniform FC1 130, FC2 76). By the sort's tiles: passes over the tile's rows.
+//
+// Needs K % 128 == 0 (four lines or more) and byte offsets of an expert's weights and of the
 // activations below 2^32.
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) quarter_kernel(GroupedParams p) {
-  const int wave = static_cast<int>(threadIdx.x) / kWave;
+constexpr int kWideRows = 32;  // rows of a pass
+
+template <bool kGated, bool kByExpert, int kBlocks = kWideRows / 16>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kBlocks == 1 ? 3 : 2))) wide_kernel(GroupedParams p) {
+  constexpr int kPassRows = 16 * kBlocks;
+  constexpr int kColumns = kGated ? 64 : 128;  // output columns of a workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int lane = lane_id();
   const int r16 = lane & 15;
   const int g = lane >> 4;
-  int64_t expert = blockIdx.x;
-  if (p.compact) {
-    __shared__ uint32_t named[kPresentExperts / 32];
-    const int64_t live = p.live_tokens != nullptr ? static_cast<int64_t>(p.live_tokens[0]) * p.top : p.routes;
-    expert = nth_named_expert<kThreads>(p.ids, p.routes, live, static_cast<int32_t>(p.local_offset),
-                                        static_cast<int32_t>(p.local_experts), static_cast<int>(blockIdx.x), named);
-    if (expert < 0) return;
+  __shared__ u32x4 regroup[kWaves][8 * 64];
+  __shared__ int32_t route_list[kByExpert ? kExpertRoutes : 1];
+  __shared__ int32_t wave_count[kWaves + 1];
+  int64_t live = 0;
+  if constexpr (kByExpert) live = p.live_tokens != nullptr ? static_cast<int64_t>(p.live_tokens[0]) * p.top : p.routes;
+
+  // The rows this workgroup takes: [row_first, row_last) of `expert`'s, found below.
+  int64_t expert, first = 0;
+  int rows = 0, row_first = 0, row_last = 0x7fffffff;
+  int64_t slice;  // the run of weight rows
+  if constexpr (kByExpert) {
+    // The first workgroups serve a column (an expert) each, slice by slice; the last ones the rows
+    // past an expert's first pass, where any has more.
+    const int b = static_cast<int>(blockIdx.x);
+    const int own = p.columns * static_cast<int>(p.out_width / kColumns);
+    const bool is_extra = b >= own;
+    const int columns = is_extra ? p.extra_columns : p.columns;
+    const int at = is_extra ? b - own : b;
+    slice = at / columns;
+    const int column = at - static_cast<int>(slice) * columns;
+    if (is_extra) {
+      const RowRun run = nth_extra_run<kThreads, kPassRows>(p.ids, p.routes, live, static_cast<int32_t>(p.local_offset),
+                                                            static_cast<int32_t>(p.local_experts), column, p.extra_columns, route_list);
+      if (run.expert < 0) return;
+      expert = run.expert;
+      row_first = run.first;
+      row_last = run.first + run.rows;
+    } else if (p.compact) {
+      __shared__ uint32_t named[kPresentExperts / 32];
+      expert = nth_named_expert<kThreads>(p.ids, p.routes, live, static_cast<int32_t>(p.local_offset),
+                                          static_cast<int32_t>(p.local_experts), column, named);
+      if (expert < 0) return;
+    } else {
+      expert = column;
+    }
+    if (!is_extra && p.extra_columns > 0) row_last = kPassRows;
+  } else {
+    const int tile = static_cast<int>(blockIdx.x);
+    slice = blockIdx.y;
+    if (tile >= p.num_tiles[0]) return;
+    expert = p.tile_to_expert[tile];
+    first = static_cast<int64_t>(tile) * kTileRows;
+    rows = p.tile_to_limit[tile] - static_cast<int>(first);
   }
-  // Row r (0..127) of the workgroup: up row slice * 64 + r, or gate row I + slice * 64 + r - 64.
-  const int64_t slice = blockIdx.y;
-  auto weight_row = [&](int r) -> int64_t { return r < 64 ? slice * 64 + r : p.out_width + slice * 64 + (r - 64); };
-  const int lines = static_cast<int>(p.K / 64);       // 128-byte lines per row
-  const int per_wave = lines / kWaves;                // this wavefront's lines: [wave * per_wave, ..)
-  const int steps = 2 * per_wave;                     // (line, half of the rows)
-  // Step t: line wave * per_wave + t / 2 of rows 64 (t % 2) + 8 i + l / 8, chunk l % 8. The rows of
-  // a half are consecutive, so load i's address is a uniform base (the expert's stack, 8 i rows on,
-  // the step's line) plus one 32-bit lane offset per half: few registers per address.
+  // Row r (0..127) of the workgroup: FC1 up row column + r, or gate row I + column + r - 64; FC2 output
+  // column `column` + r.
+  const int64_t column = slice * kColumns;
+  auto weight_row = [&](int r) -> int64_t {
+    if constexpr (kGated) return r < 64 ? column + r : p.out_width + column + (r - 64);
+    else return column + r;
+  };
+  const int lines = static_cast<int>(p.K / 64);  // 128-byte lines per row
+  const int line_first = wave * lines / kWaves;  // this wavefront's lines
+  const int line_count = (wave + 1) * lines / kWaves - line_first;
+  // Line l of half h: rows 64 h + 8 i + lane / 8, chunk lane % 8.
   expert = __builtin_amdgcn_readfirstlane(static_cast<int>(expert));
-  const uint8_t *wbase = reinterpret_cast<const uint8_t *>(p.weights + expert * p.n_total * p.K);
-  const int64_t row_bytes = p.K * 2;
+  const uint32_t row_bytes = static_cast<uint32_t>(p.K * 2);
+  const BufferBase weights = buffer_base(p.weights + expert * p.n_total * p.K, static_cast<uint32_t>(p.n_total) * row_bytes);
   uint32_t half_off[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
-    half_off[h] = static_cast<uint32_t>(weight_row(64 * h + lane / 8) * row_bytes + wave * per_wave * 128 + (lane & 7) * 16);
-  struct Step {
+    half_off[h] = static_cast<uint32_t>(weight_row(64 * h + lane / 8)) * row_bytes + line_first * 128 + (lane & 7) * 16;
+  struct Half {
     u32x4 lines[8];
   };
-  auto load_step = [&](Step &st, int t) {
-    const int h = t & 1;
-    const uint8_t *line = wbase + static_cast<int64_t>(t >> 1) * 128;
+  auto load_half = [&](Half &st, int line, int h) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      st.lines[i] = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4 *>(line + static_cast<int64_t>(i) * 8 * row_bytes + half_off[h]));
+      st.lines[i] = buffer_load16<true>(weights, half_off[h], static_cast<uint32_t>(line) * 128 + i * 8 * row_bytes);
   };
-  Step even, odd;
-  const FirstRouteIds first_ids = load_first_route_ids<kWaves>(p.ids, p.routes);
-  load_step(even, 0);  // no dependence on the routes: out before the scan (after the ids it reads)
+  Half even, odd;
+  FirstRouteIds first_ids;
+  if constexpr (kByExpert) first_ids = load_first_route_ids<kWaves>(p.ids, p.routes);
+  load_half(even, 0, 0);  // no dependence on the routes: out before the scan (after the ids it reads)
 
-  __shared__ u32x4 regroup[kWaves][8 * 64];
-  __shared__ int32_t route_list[kExpertRoutes];
-  __shared__ int32_t wave_count[kWaves + 1];
-  const int64_t live = p.live_tokens != nullptr ? static_cast<int64_t>(p.live_tokens[0]) * p.top : p.routes;
-  const int rows = list_expert_routes<kWaves>(p.ids, p.routes, live, static_cast<int32_t>(expert + p.local_offset),
-                                              route_list, wave_count, &first_ids);
-  if (rows == 0) return;
+  if constexpr (kByExpert) {
+    rows = list_expert_routes<kWaves>(p.ids, p.routes, live, static_cast<int32_t>(expert + p.local_offset),
+                                      route_list, wave_count, &first_ids);
+    if (rows == 0) return;
+  }
   auto listed = [&](int m) -> int64_t { return listed_route<kWaves>(route_list, wave_count, p.routes, m); };
+  // FC2 by tiles reads the tile's own rows: addressed from the tile's first row.
+  const BufferBase act = buffer_base(p.act + (kByExpert || kGated ? 0 : first * p.K), 0xffffffffu);
+  const int row_end = min(rows, row_last);
 
-  for (int pass = 0; pass < rows; pass += 16) {
-    const int m = pass + r16;
-    const bool valid = m < rows;
-    const int64_t source = valid ? listed(m) / p.top : 0;
-    // Rows past the expert's routes read row 0 (never stored).
-    const uint32_t a_off = static_cast<uint32_t>((source * p.K + static_cast<int64_t>(wave) * per_wave * 64 + g * 8) * 2);
-    const uint8_t *act = reinterpret_cast<const uint8_t *>(p.act);
-    floatx4 acc[8];
+  for (int pass = row_first; pass < row_end; pass += kPassRows) {
+    uint32_t a_off[kBlocks];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    u32x4 x[2][2];  // [line parity][K step of 32]: this lane's 8 elements of each
-    auto load_x = [&](int line, u32x4 (&into)[2]) {
-      into[0] = *reinterpret_cast<const u32x4 *>(act + static_cast<int64_t>(line) * 128 + a_off);
-      into[1] = *reinterpret_cast<const u32x4 *>(act + static_cast<int64_t>(line) * 128 + 64 + a_off);
+    for (int mb = 0; mb < kBlocks; ++mb) {
+      const int m = pass + 16 * mb + r16;
+      int64_t source = 0;  // rows past the expert's routes read row 0 (never stored)
+      if (m < rows) {
+        if constexpr (kByExpert) source = kGated ? listed(m) / p.top : listed(m);
+        else source = kGated ? p.permuted_to_expanded[first + m] / p.top : m;
+      }
+      a_off[mb] = static_cast<uint32_t>((source * p.K + static_cast<int64_t>(line_first) * 64 + g * 8) * 2);
+    }
+    floatx4 acc[8][kBlocks];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb) acc[j][mb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    struct Acts {
+      u32x4 x[kBlocks][2];  // [row block][K step of 32]: this lane's 8 elements of each
     };
-    auto compute = [&](const Step &st, int t, const u32x4 (&xs)[2]) {
+    Acts xa, xb;
+    auto load_x = [&](Acts &into, int line) {
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          into.x[mb][ks] = buffer_load16<false>(act, a_off[mb], static_cast<uint32_t>(line) * 128 + 64 * ks);
+    };
+    auto compute = [&](const Half &st, int h, const Acts &xs) {
       {
         const int row = lane >> 3, piece = lane & 7;
 #pragma unroll
         for (int i = 0; i < 8; ++i) regroup[wave][i * 64 + row * 8 + (piece ^ row)] = st.lines[i];
       }
-      const int h = t & 1;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int i = 2 * j + (r16 >> 3), rr = r16 & 7, q = 4 * ks + g;
           const u32x4 w = regroup[wave][i * 64 + rr * 8 + (q ^ rr)];
-          acc[4 * h + j] = mfma_16x16x32_bf16(w, xs[ks], acc[4 * h + j]);
+#pragma unroll
+          for (int mb = 0; mb < kBlocks; ++mb) acc[4 * h + j][mb] = mfma_16x16x32_bf16(w, xs.x[mb][ks], acc[4 * h + j][mb]);
         }
     };
-    if (pass > 0) load_step(even, 0);
-    load_x(0, x[0]);
-    // Steps in pairs (both halves of one line); the next pair's loads go out before this pair's
-    // computes wait, all unconditionally in the steady walk.
-    int t = 0;
-    for (; t + 2 < steps; t += 2) {
-      load_step(odd, t + 1);
-      load_x((t >> 1) + 1, x[1]);
-      compute(even, t, x[0]);
-      load_step(even, t + 2);
-      compute(odd, t + 1, x[0]);
-      x[0][0] = x[1][0];
-      x[0][1] = x[1][1];
+    if (pass > row_first) load_half(even, 0, 0);
+    load_x(xa, 0);
+    load_half(odd, 0, 1);
+    // A line that has a next one: its halves' buffers are filled with the next line's as soon as
+    // they are consumed, all unconditionally, so each wait counts exactly the loads still in flight.
+    auto line = [&](int l, const Acts &now, Acts &next) {
+      load_x(next, l + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(even, 0, now);
+      __builtin_amdgcn_sched_barrier(0);
+      load_half(even, l + 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(odd, 1, now);
+      __builtin_amdgcn_sched_barrier(0);
+      load_half(odd, l + 1, 1);
+    };
+    auto last_line = [&](const Acts &now) {
+      compute(even, 0, now);
+      compute(odd, 1, now);
+    };
+    int l = 0;
+    for (; l + 2 < line_count; l += 2) {
+      line(l, xa, xb);
+      line(l + 1, xb, xa);
     }
-    load_step(odd, t + 1);
-    compute(even, t, x[0]);
-    compute(odd, t + 1, x[0]);
+    if (l + 1 < line_count) {
+      line(l, xa, xb);
+      last_line(xb);
+    } else {
+      last_line(xa);
+    }
 
-    // The four quarters' partial sums, added in wave order; each wavefront's go through its own
-    // regroup buffer (8 x 64 floatx4, the buffer's size), which it no longer reads.
+    // The wavefronts' partial sums, added in wave order, one row block at a time; each wavefront's go
+    // through its own regroup buffer (8 x 64 floatx4, the buffer's size), which it no longer reads.
+    // FC1: wavefront w adds up set w and gate set w + 4 (16 gated columns); FC2: sets 2 w, 2 w + 1.
     auto partial = [&](int w, int j) -> floatx4 & { return reinterpret_cast<floatx4 *>(regroup[w])[j * kWave + lane]; };
+    auto total = [&](int j) {
+      floatx4 sum = partial(0, j);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) partial(wave, j) = acc[j];
-    __syncthreads();
-    floatx4 up = partial(0, wave), gated = partial(0, wave + 4);
+      for (int w = 1; w < kWaves; ++w) sum += partial(w, j);
+      return sum;
+    };
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
-      up += partial(w, wave);
-      gated += partial(w, wave + 4);
+    for (int mb = 0; mb < kBlocks; ++mb) {
+      if (pass + 16 * mb >= rows) break;  // (uniform)
+      if (mb > 0) __syncthreads();        // the block before is summed
+#pragma unroll
+      for (int j = 0; j < 8; ++j) partial(wave, j) = acc[j][mb];
+      __syncthreads();
+      const floatx4 sum0 = total(kGated ? wave : 2 * wave), sum1 = total(kGated ? wave + 4 : 2 * wave + 1);
+      const int m = pass + 16 * mb + r16;
+      if (m < rows) {
+        uint16_t *row = p.out + (kByExpert ? listed(m) : first + m) * p.out_width + column + 4 * g;
+        if constexpr (kGated) {
+          floatx4 h;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) h[i] = gate(sum1[i], p.activation) * sum0[i];
+          store_bf16x4(row + wave * 16, h);
+        } else {
+          store_bf16x4(row + wave * 32, sum0);
+          store_bf16x4(row + wave * 32 + 16, sum1);
+        }
+      }
     }
-    __syncthreads();  // the next pass regroups over the partial sums
-    if (valid) {
-      floatx4 hv;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) hv[i] = gate(gated[i], p.activation) * up[i];
-      store_bf16x4(p.out + listed(m) * p.out_width + slice * 64 + wave * 16 + 4 * g, hv);
-    }
+    __syncthreads();  // the next pass's lines overwrite the partial sums
   }
 }
 
@@ -545,11 +638,31 @@ __global__ void __launch_bounds__(kThreads) tiled_kernel(GroupedParams p) {
   }
 }
 
-/// The stream kernel serves batches whose experts average fewer rows than this.
+/// The stream and wide kernels serve batches whose experts average fewer rows than this.
 constexpr int64_t kStreamRowsPerExpert = 24;
 
+/// FC2 by expert with at most this many rows per expert on average stays on the stream kernel,
+/// whose workgroups need no exchange of partial sums (30B: T=5 21.1 us against 23.4 on the wide
+/// kernel, T=64 62.0 against 62.5 - with Zipf routing, where some experts have more than 16 rows, 86
+/// against 50 - and T=128 70 against 65).
+constexpr int64_t kWideFc2RowsPerExpert = 2;
+
+/// FC1 by expert with at most this many rows per expert on average: 16 rows a pass, whose fewer
+/// registers leave three waves per SIMD (30B: T=32 104 us against 107; T=64 117.6 against 118.3, but
+/// 150 against 98 with Zipf routing, where some experts have more rows than that).
+constexpr int64_t kWideOneBlockRowsPerExpert = 2;
+
+/// By the sort's tiles: workgroups below which the wide kernel is not worth its exchange.
+constexpr int64_t kWideWorkgroups = 170;
+
+/// Whether the wide kernel serves the product over `act_rows` activation rows.
+bool wide_fits(const GroupedParams &p, int64_t act_rows) {
+  constexpr int64_t kOffsetRange = int64_t{1} << 32;
+  return p.K % 128 == 0 && p.K / 64 >= kWaves && p.n_total * p.K * 2 < kOffsetRange && act_rows * p.K * 2 < kOffsetRange;
+}
+
 template <bool kGated>
-void launch_grouped(const GroupedParams &p, int64_t max_tiles, bool stream_path, bool one_pass, hipStream_t s) {
+void launch_grouped(const GroupedParams &p, int64_t max_tiles, int64_t act_rows, bool stream_path, bool few_rows, hipStream_t s) {
   if (!stream_path && (pair_fits<pair::Bf16>(kGated, p.K, p.out_width, 0) || prefill_fits<prefill::Bf16, kGated>(p.K, p.out_width))) {
     PrefillParams q{};
     q.act = reinterpret_cast<const uint8_t *>(p.act);
@@ -570,8 +683,12 @@ void launch_grouped(const GroupedParams &p, int64_t max_tiles, bool stream_path,
   }
   const int64_t slices = kGated ? p.out_width / 64 : ceil_div<int64_t>(p.out_width, 128);
   const dim3 grid(static_cast<uint32_t>(max_tiles), static_cast<uint32_t>(slices));
-  if (stream_path && one_pass) hipLaunchKernelGGL((stream_kernel<kGated, 1>), grid, dim3(kThreads), 0, s, p);
-  else if (stream_path) hipLaunchKernelGGL((stream_kernel<kGated, 2>), grid, dim3(kThreads), 0, s, p);
+  // Below two wide workgroups per three CUs the stream kernel, whose workgroups end without an exchange
+  // of partial sums (30B T=1: FC1 14.3 us against 16.6; 235B T=1, 192 workgroups: 35.8 against 34.2).
+  if (stream_path && max_tiles * slices >= kWideWorkgroups && (kGated || (!few_rows && p.out_width % 128 == 0)) &&
+      wide_fits(p, act_rows))
+    hipLaunchKernelGGL((wide_kernel<kGated, false>), grid, dim3(kThreads), 0, s, p);
+  else if (stream_path) hipLaunchKernelGGL((stream_kernel<kGated, false>), grid, dim3(kThreads), 0, s, p);
   else hipLaunchKernelGGL(tiled_kernel<kGated>, grid, dim3(kThreads), 0, s, p);
 }
 
@@ -580,10 +697,10 @@ void launch_grouped(const GroupedParams &p, int64_t max_tiles, bool stream_path,
 
 namespace uniserve {
 
-bool expert_stream_fits(int64_t routes, int64_t local_experts, int64_t K, int64_t out_width, bool gated) {
+bool expert_stream_fits(int64_t routes, int64_t experts, int64_t local_experts, int64_t K, int64_t out_width, bool gated) {
   // Fewer routes than local experts: a compact grid (a workgroup column per route, each finding
   // the n-th named expert), which tells at most kPresentExperts experts apart.
-  return routes >= 1 && routes <= kExpertRoutes && routes < kStreamRowsPerExpert * local_experts &&
+  return routes >= 1 && routes <= kExpertRoutes && routes < kStreamRowsPerExpert * experts &&
          (routes >= local_experts || local_experts <= kPresentExperts) && K % 128 == 0 &&
          (gated ? out_width % 64 == 0 : out_width % 128 == 0) && local_experts <= 0x7fffffffLL;
 }
@@ -604,18 +721,24 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
   p.local_offset = e.local_offset;
   p.local_experts = e.local_experts;
   p.compact = e.routes < e.local_experts ? 1 : 0;
-  const bool one_pass = e.routes <= kOnePassRowsPerExpert * e.local_experts;
   const int64_t slices = gated ? e.out_width / 64 : e.out_width / 128;
   const dim3 grid(static_cast<uint32_t>(p.compact ? e.routes : e.local_experts), static_cast<uint32_t>(slices));
-  constexpr int64_t kOffsetRange = int64_t{1} << 32;  // the quarter kernel's 32-bit byte offsets
-  if (gated && e.K % 256 == 0 && e.n_total * e.K * 2 < kOffsetRange && e.routes * e.K * 2 < kOffsetRange) {
-    hipLaunchKernelGGL(quarter_kernel, grid, dim3(kThreads), 0, stream, p);
+  if (wide_fits(p, e.routes) && (gated || e.routes > kWideFc2RowsPerExpert * e.experts)) {
+    // An expert with more rows than one pass takes leaves the rest to workgroups of their own (with
+    // one column per expert that may have any: nth_extra_run).
+    const int64_t extra = (e.routes - 1) / kWideRows;
+    p.extra_columns = p.compact || e.routes <= 2 * kWideRows * e.top
+                          ? 0 : static_cast<int32_t>(extra < e.local_experts ? extra : e.local_experts);
+    p.columns = static_cast<int32_t>(grid.x);
+    const dim3 wide_grid(static_cast<uint32_t>((p.columns + p.extra_columns) * slices));
+    if (gated && e.routes <= kWideOneBlockRowsPerExpert * e.experts)
+      hipLaunchKernelGGL((wide_kernel<true, true, 1>), wide_grid, dim3(kThreads), 0, stream, p);
+    else if (gated) hipLaunchKernelGGL((wide_kernel<true, true>), wide_grid, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((wide_kernel<false, true>), wide_grid, dim3(kThreads), 0, stream, p);
     return;
   }
-  if (gated && one_pass) hipLaunchKernelGGL((stream_kernel<true, 1, true>), grid, dim3(kThreads), 0, stream, p);
-  else if (gated) hipLaunchKernelGGL((stream_kernel<true, 2, true>), grid, dim3(kThreads), 0, stream, p);
-  else if (one_pass) hipLaunchKernelGGL((stream_kernel<false, 1, true>), grid, dim3(kThreads), 0, stream, p);
-  else hipLaunchKernelGGL((stream_kernel<false, 2, true>), grid, dim3(kThreads), 0, stream, p);
+  if (gated) hipLaunchKernelGGL((stream_kernel<true, true>), grid, dim3(kThreads), 0, stream, p);
+  else hipLaunchKernelGGL((stream_kernel<false, true>), grid, dim3(kThreads), 0, stream, p);
 }
 
 int32_t gather_gemm_bf16(const uniserve_gather_call *call, int32_t activation, void *stream) {
@@ -665,8 +788,7 @@ int32_t gather_gemm_bf16(const uniserve_gather_call *call, int32_t activation, v
     p.activation = activation;
     const bool stream_path = call->tokens * call->top < kStreamRowsPerExpert * call->experts &&
                              call->hidden_size % 128 == 0;
-    launch_grouped<true>(p, max_tiles, stream_path, call->tokens * call->top <= kOnePassRowsPerExpert * call->experts,
-                         static_cast<hipStream_t>(stream));
+    launch_grouped<true>(p, max_tiles, call->tokens, stream_path, false, static_cast<hipStream_t>(stream));
     return launched(call, "gather_gemm");
   });
 }
@@ -720,7 +842,7 @@ extern "C" int32_t uniserve_route_gemm(const uniserve_route_call *call, void *st
     const int64_t routes_bound = call->permuted_rows - (kTileRows - 1) * call->experts;
     const bool stream_path = routes_bound < kStreamRowsPerExpert * call->experts &&
                              call->intermediate % 128 == 0;
-    launch_grouped<false>(p, max_tiles, stream_path, routes_bound <= kOnePassRowsPerExpert * call->experts,
+    launch_grouped<false>(p, max_tiles, kTileRows, stream_path, routes_bound <= kWideFc2RowsPerExpert * call->experts,
                           static_cast<hipStream_t>(stream));
     return launched(call, "route_gemm");
   });

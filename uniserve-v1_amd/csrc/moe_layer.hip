@@ -344,9 +344,10 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
     const int64_t routes = call->tokens * call->top;
     const bool front = front_fits(call->tokens, call->experts, call->hidden_size, call->top, local_experts);
     const bool by_expert = front &&
-                           expert_stream_fits(routes, local_experts, call->hidden_size, call->intermediate, true) &&
-                           expert_stream_fits(routes, local_experts, call->intermediate, call->hidden_size, false) &&
+                           expert_stream_fits(routes, call->experts, local_experts, call->hidden_size, call->intermediate, true) &&
+                           expert_stream_fits(routes, call->experts, local_experts, call->intermediate, call->hidden_size, false) &&
                            (!mx || (call->hidden_size % 256 == 0 && call->intermediate % 256 == 0));
+    if (by_expert) v.route_scales = 0;  // (rows at expanded positions: no permuted rows to lay scales out by)
 
     // e4m3 and MXFP4 at those sizes: the front end also quantises the hidden rows (QUANTIZE_HIDDEN
     // then launches nothing).
@@ -531,6 +532,7 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
       e.top = call->top;
       e.local_offset = call->local_offset;
       e.local_experts = local_experts;
+      e.experts = call->experts;
       e.activation = activation;
       if (want(UNISERVE_MOE_LAYER_GATHER)) {
         ExpertStream fc1 = e;
