@@ -44,6 +44,7 @@ constexpr int kWaveRows = 64;                // weight rows per wavefront
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * kWave;
 constexpr int kSliceRows = kWaves * kWaveRows;
+constexpr int kResident = 512;               // workgroups resident at a time: two on each of 256 CUs
 constexpr int kActStages = 3;
 constexpr int kTokenBlocks = kRows / 16;
 constexpr int kWeightLoads = kWaveRows / 8;  // 16-byte DMA instructions per wave per stage (8 rows each)
@@ -120,7 +121,8 @@ constexpr int lds_bytes() {
 }
 
 /// e4m3 needs route-major activation scales (p.scale_rows >= the tiles' rows).
-template <class F, bool kGated>
+/// kSpread: the items' K walks may start at different stages.
+template <class F, bool kGated, bool kSpread>
 __global__ void __launch_bounds__(kThreads, 2) pair_kernel(PrefillParams p) {
   using prefill::dma16;
   using prefill::dma16_after_lds_reads;
@@ -216,28 +218,49 @@ __global__ void __launch_bounds__(kThreads, 2) pair_kernel(PrefillParams p) {
     asm volatile("" ::"v"(sw_lanes[0]), "v"(sw_lanes[1]));
   }
 
-  // Weights of stage k, the h-th of `parts` equal runs of the eight instructions; `after_reads`:
+  // The K stage of the loop's step k. Where the live items are one to four rounds of resident
+  // workgroups, each (expert, slice) starts its walk at a stage of its own and wraps around:
+  // workgroups that start together would otherwise all read the same 128-byte column of their rows at
+  // a time, which with row strides of whole 4 KB falls on few HBM channels. (The tiles of an expert
+  // share their starts, and so their weights in L2.) A Weyl sequence over (expert, slice) spreads the
+  // starts evenly. 30B bf16 near-uniform T=450 FC1 188 -> 159 us, T=1024 194 -> 167; 235B e4m3 T=640
+  // 335 -> 297. With more rounds the items drift apart by themselves and the slices of a tile gain
+  // from reading its activation rows together (30B bf16 T=8192: 460 us, spread 474); with less than
+  // one, likewise (sixteen 235B experts, bf16 T=1024: 134, spread 142).
+  int start = 0;
+  if constexpr (kSpread) {
+    const int live_items = p.num_tiles[0] * p.slices;
+    const uint32_t walk = (static_cast<uint32_t>(expert) * static_cast<uint32_t>(p.slices) + static_cast<uint32_t>(slice)) * 0x9e3779b1u;
+    if (live_items >= kResident && live_items <= 4 * kResident)
+      start = __builtin_amdgcn_readfirstlane(static_cast<int>(__umulhi(walk, static_cast<uint32_t>(stages))));
+  }
+  auto stage_of = [&](int k) {
+    if constexpr (!kSpread) return k;
+    return k + start < stages ? k + start : k + start - stages;
+  };
+
+  // Weights of a K stage, the h-th of `parts` equal runs of the eight instructions; `after_reads`:
   // the wave just read its rows of the buffer, and the first DMA waits for those LDS reads
   // (lgkmcnt 0) before it may overwrite them.
-  auto issue_weights = [&](int k, int h, bool after_reads, int parts = 2) {
+  auto issue_weights = [&](int stage, int h, bool after_reads, int parts = 2) {
     const uint32_t weight_lds = lds_address(sh.weights[wave]);
 #pragma unroll
     for (int j = 0; j < kWeightLoads / parts; ++j) {
       const int i = h * (kWeightLoads / parts) + j;
-      const uint8_t *base = w_base[i / 4] + static_cast<int64_t>(k) * 128 + static_cast<int64_t>(i % 4) * 8 * row_bytes;
+      const uint8_t *base = w_base[i / 4] + static_cast<int64_t>(stage) * 128 + static_cast<int64_t>(i % 4) * 8 * row_bytes;
       const uint32_t lane_offset = w_lane + ((w_chunk ^ static_cast<uint32_t>(4 * (i & 1))) << 4);
       const uint32_t dst = __builtin_amdgcn_readfirstlane(weight_lds + i * kWave * 16);
       if (i == 0 && after_reads) dma16_after_lds_reads(base, lane_offset, dst);
       else dma16(base, lane_offset, dst);
     }
   };
-  // Activations of stage k, instructions kActLoads / 2 h ..
-  auto issue_act = [&](int k, int h) {
+  // Activations of a K stage, step k's, instructions kActLoads / 2 h ..
+  auto issue_act = [&](int k, int stage, int h) {
     const uint32_t act_lds = lds_address(sh.act[k % kActStages] + wave * kActLoads * kWave);
 #pragma unroll
     for (int j = 0; j < kActLoads / 2; ++j) {
       const int i = h * (kActLoads / 2) + j;
-      dma16(act_tile + static_cast<int64_t>(k) * 128, a_off[i], __builtin_amdgcn_readfirstlane(act_lds + i * kWave * 16));
+      dma16(act_tile + static_cast<int64_t>(stage) * 128, a_off[i], __builtin_amdgcn_readfirstlane(act_lds + i * kWave * 16));
     }
   };
 
@@ -258,16 +281,16 @@ __global__ void __launch_bounds__(kThreads, 2) pair_kernel(PrefillParams p) {
   // the barrier for the other wavefronts' activation rows. (At least three stages: pair_fits.) ----
   constexpr int kLast = kActLoads;  // loads of the farthest group
   float sx[kTokenBlocks];
-  issue_act(0, 0);
-  issue_act(0, 1);
-  issue_weights(0, 0, false);
-  issue_weights(0, 1, false);
+  issue_act(0, start, 0);
+  issue_act(0, start, 1);
+  issue_weights(start, 0, false);
+  issue_weights(start, 1, false);
   if constexpr (F::kScaled) {
-    load_scales_half<0>(sx, scale_table, sx_off);
-    load_scales_half<1>(sx, scale_table, sx_off);
+    load_scales_half<0>(sx, scale_table + start * sx_stage, sx_off);
+    load_scales_half<1>(sx, scale_table + start * sx_stage, sx_off);
   }
-  issue_act(1, 0);
-  issue_act(1, 1);
+  issue_act(1, stage_of(1), 0);
+  issue_act(1, stage_of(1), 1);
   if constexpr (F::kScaled) wait_loads_and_scales<kLast>(sx);
   for (int k = 0; k < stages; ++k) {
     prefill::wait_loads_but<kLast>();
@@ -277,23 +300,24 @@ __global__ void __launch_bounds__(kThreads, 2) pair_kernel(PrefillParams p) {
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb) wf[jb] = fragment(sh.weights[wave], jb * 16 + r16, g);
     const int act_next = min(k + 2, stages - 1);
-    const int next = min(k + 1, stages - 1);
+    const int next_stage = stage_of(min(k + 1, stages - 1));
+    const int act_stage = stage_of(act_next);
     // The loads issued before token block tb's MFMAs: two weight instructions before each of the
     // first four blocks, then the scales, then the activations.
     auto issue_part = [&](int tb) {
-      if (tb < 4) issue_weights(next, tb, tb == 0, 4);
+      if (tb < 4) issue_weights(next_stage, tb, tb == 0, 4);
       constexpr int kActAt = F::kScaled ? 6 : 4;
       if constexpr (F::kScaled) {
-        if (tb == 4) load_scales_half<0>(sx, scale_table + next * sx_stage, sx_off);
-        if (tb == 5) load_scales_half<1>(sx, scale_table + next * sx_stage, sx_off);
+        if (tb == 4) load_scales_half<0>(sx, scale_table + next_stage * sx_stage, sx_off);
+        if (tb == 5) load_scales_half<1>(sx, scale_table + next_stage * sx_stage, sx_off);
       }
-      if (tb == kActAt) issue_act(act_next, 0);
-      if (tb == kActAt + 1) issue_act(act_next, 1);
+      if (tb == kActAt) issue_act(act_next, act_stage, 0);
+      if (tb == kActAt + 1) issue_act(act_next, act_stage, 1);
     };
 
     if constexpr (F::kScaled) {
-      const float sw0 = __int_as_float(__builtin_amdgcn_readlane(sw_lanes[0], k));
-      const float sw1 = __int_as_float(__builtin_amdgcn_readlane(sw_lanes[1], k));
+      const float sw0 = __int_as_float(__builtin_amdgcn_readlane(sw_lanes[0], stage_of(k)));
+      const float sw1 = __int_as_float(__builtin_amdgcn_readlane(sw_lanes[1], stage_of(k)));
       float sc[kTokenBlocks][2];
 #pragma unroll
       for (int tb = 0; tb < kTokenBlocks; ++tb) {
@@ -530,8 +554,15 @@ inline void launch_pair(PrefillParams p, bool gated, int64_t max_tiles, hipStrea
   p.groups_per_xcd = static_cast<int32_t>(ceil_div<int64_t>(ceil_div<int64_t>(max_tiles, group), 8));
   const dim3 grid(static_cast<uint32_t>(static_cast<int64_t>(p.groups_per_xcd) * group * p.slices * 8));
   const dim3 block(static_cast<uint32_t>(pair::kThreads));
-  if (gated) hipLaunchKernelGGL((pair::pair_kernel<F, true>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((pair::pair_kernel<F, false>), grid, block, 0, stream, p);
+  // Up to six rounds of resident workgroups if every tile is live: the kernel that may spread its K
+  // walks (the live tiles, which only the device knows, decide). Above, without the stage arithmetic
+  // (235B e4m3 T=4096 layer 1111 us, 1124 with it).
+  const bool spread = max_tiles * p.slices <= 6 * pair::kResident;
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, p); };
+  if (gated && spread) go(pair::pair_kernel<F, true, true>);
+  else if (gated) go(pair::pair_kernel<F, true, false>);
+  else if (spread) go(pair::pair_kernel<F, false, true>);
+  else go(pair::pair_kernel<F, false, false>);
 }
 
 }  // namespace uniserve
