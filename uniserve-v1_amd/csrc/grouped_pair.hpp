@@ -556,8 +556,11 @@ inline void launch_pair(PrefillParams p, bool gated, int64_t max_tiles, hipStrea
   const dim3 block(static_cast<uint32_t>(pair::kThreads));
   // Up to six rounds of resident workgroups if every tile is live: the kernel that may spread its K
   // walks (the live tiles, which only the device knows, decide). Above, without the stage arithmetic
-  // (235B e4m3 T=4096 layer 1111 us, 1124 with it).
-  const bool spread = max_tiles * p.slices <= 6 * pair::kResident;
+  // (235B e4m3 T=4096 layer 1102 us, 1124 with it). e4m3 rows, half as long, only at whole 4 KB: the
+  // 2 KB rows of a 30B FC1 gain nothing (T=512..2048 within 1%), and keep the sums of the stand-alone
+  // products.
+  const bool spread = max_tiles * p.slices <= 6 * pair::kResident &&
+                      (!F::kScaled || p.K * F::kElementBytes % 4096 == 0);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, p); };
   if (gated && spread) go(pair::pair_kernel<F, true, true>);
   else if (gated) go(pair::pair_kernel<F, true, false>);
