@@ -136,6 +136,10 @@ buffer_load16(BufferBase base, uint32_t lane_offset, uint32_t offset) {
   return __builtin_amdgcn_raw_buffer_load_b128(base, lane_offset, offset, kOnce ? 2 : 0);
 }
 
+__device__ __forceinline__ float buffer_load_f32(BufferBase base, uint32_t lane_offset, uint32_t offset) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(base, lane_offset, offset, 0));
+}
+
 // ---- MFMA operands ------------------------------------------------------------------------------------
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

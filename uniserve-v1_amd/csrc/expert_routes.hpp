@@ -184,6 +184,51 @@ __device__ __forceinline__ RowRun nth_extra_run(const int32_t *ids, int64_t rout
   return found;
 }
 
+/// What one workgroup of a wide kernel (a one-dimensional grid of (columns + extra_columns) * slices)
+/// serves: rows [row_first, row_last) of `expert`'s, its `slice`-th run of weight rows.
+struct ColumnWork {
+  int32_t expert;  ///< local expert, or -1: nothing
+  int32_t slice;
+  int32_t row_first, row_last;
+};
+
+/// The first columns * slices workgroups serve a column - an expert, or with `compact` the n-th named
+/// one - each, slice by slice, and the last extra_columns * slices the rows past an expert's first
+/// kPassRows, where any has more (nth_extra_run). Every thread of the workgroup calls it; `list` holds
+/// local_experts words and is free again when it returns.
+template <int kThreads, int kPassRows, class Params>
+__device__ __forceinline__ ColumnWork column_work(const Params &p, int64_t live, int slices, int32_t *list) {
+  __shared__ uint32_t named[kPresentExperts / 32];
+  ColumnWork work{-1, 0, 0, 0x7fffffff};
+  const int b = static_cast<int>(blockIdx.x);
+  const int own = p.columns * slices;
+  const bool is_extra = b >= own;
+  const int columns = is_extra ? p.extra_columns : p.columns;
+  const int at = is_extra ? b - own : b;
+  work.slice = at / columns;
+  const int column = at - work.slice * columns;
+  const int32_t offset = static_cast<int32_t>(p.local_offset), experts = static_cast<int32_t>(p.local_experts);
+  if (is_extra) {
+    const RowRun run = nth_extra_run<kThreads, kPassRows>(p.ids, p.routes, live, offset, experts, column, p.extra_columns, list);
+    work.expert = run.expert;
+    work.row_first = run.first;
+    work.row_last = run.first + run.rows;
+    return work;
+  }
+  work.expert = p.compact ? nth_named_expert<kThreads>(p.ids, p.routes, live, offset, experts, column, named) : column;
+  if (p.extra_columns > 0) work.row_last = kPassRows;
+  return work;
+}
+
+/// The extra columns a launch needs: one per run of `pass_rows` that may lie past an expert's first
+/// (never more than the experts), none for a compact grid or where no expert is likely to have more
+/// than two passes of rows (`tokens`, unless the slot map names a slot twice).
+inline int32_t extra_columns(int64_t routes, int64_t top, int64_t local_experts, bool compact, int64_t pass_rows) {
+  const int64_t runs = (routes - 1) / pass_rows;
+  if (compact || routes <= 2 * pass_rows * top) return 0;
+  return static_cast<int32_t>(runs < local_experts ? runs : local_experts);
+}
+
 /// Row m of the list (m < the total).
 template <int kWaves>
 __device__ __forceinline__ int64_t listed_route(const int32_t *list, const int32_t *counts, int64_t routes, int m) {

@@ -149,7 +149,10 @@ struct GroupedFp8Params {
   int64_t routes;
   int64_t local_offset;
   int64_t local_experts;
+  int64_t experts;              ///< the router's (routes / experts: the rows an expert expects)
   int32_t compact;              ///< workgroup x serves the x-th named local expert
+  int32_t columns;              ///< wide kernel: workgroup columns (experts, or routes if compact)
+  int32_t extra_columns;        ///< wide kernel: columns past those, for rows past an expert's first pass
 };
 
 void launch_quantize_fp8(const void *input, bool input_f32, uint8_t *out, float *scales,

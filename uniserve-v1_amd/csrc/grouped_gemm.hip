@@ -328,31 +328,12 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(k
   int rows = 0, row_first = 0, row_last = 0x7fffffff;
   int64_t slice;  // the run of weight rows
   if constexpr (kByExpert) {
-    // The first workgroups serve a column (an expert) each, slice by slice; the last ones the rows
-    // past an expert's first pass, where any has more.
-    const int b = static_cast<int>(blockIdx.x);
-    const int own = p.columns * static_cast<int>(p.out_width / kColumns);
-    const bool is_extra = b >= own;
-    const int columns = is_extra ? p.extra_columns : p.columns;
-    const int at = is_extra ? b - own : b;
-    slice = at / columns;
-    const int column = at - static_cast<int>(slice) * columns;
-    if (is_extra) {
-      const RowRun run = nth_extra_run<kThreads, kPassRows>(p.ids, p.routes, live, static_cast<int32_t>(p.local_offset),
-                                                            static_cast<int32_t>(p.local_experts), column, p.extra_columns, route_list);
-      if (run.expert < 0) return;
-      expert = run.expert;
-      row_first = run.first;
-      row_last = run.first + run.rows;
-    } else if (p.compact) {
-      __shared__ uint32_t named[kPresentExperts / 32];
-      expert = nth_named_expert<kThreads>(p.ids, p.routes, live, static_cast<int32_t>(p.local_offset),
-                                          static_cast<int32_t>(p.local_experts), column, named);
-      if (expert < 0) return;
-    } else {
-      expert = column;
-    }
-    if (!is_extra && p.extra_columns > 0) row_last = kPassRows;
+    const ColumnWork work = column_work<kThreads, kPassRows>(p, live, static_cast<int>(p.out_width / kColumns), route_list);
+    if (work.expert < 0) return;
+    expert = work.expert;
+    slice = work.slice;
+    row_first = work.row_first;
+    row_last = work.row_last;
   } else {
     const int tile = static_cast<int>(blockIdx.x);
     slice = blockIdx.y;
@@ -726,9 +707,7 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
   if (wide_fits(p, e.routes) && (gated || e.routes > kWideFc2RowsPerExpert * e.experts)) {
     // An expert with more rows than one pass takes leaves the rest to workgroups of their own (with
     // one column per expert that may have any: nth_extra_run).
-    const int64_t extra = (e.routes - 1) / kWideRows;
-    p.extra_columns = p.compact || e.routes <= 2 * kWideRows * e.top
-                          ? 0 : static_cast<int32_t>(extra < e.local_experts ? extra : e.local_experts);
+    p.extra_columns = extra_columns(e.routes, e.top, e.local_experts, p.compact != 0, kWideRows);
     p.columns = static_cast<int32_t>(grid.x);
     const dim3 wide_grid(static_cast<uint32_t>((p.columns + p.extra_columns) * slices));
     if (gated && e.routes <= kWideOneBlockRowsPerExpert * e.experts)

@@ -370,6 +370,221 @@ __global__ void __launch_bounds__(kWaves * kWave) stream_fp8_kernel(GroupedFp8Pa
   }
 }
 
+// ---- wide kernel (decode and continuous batches, expert-major) -----------------------------------------------
+//
+// The bf16 wide kernel's form (grouped_gemm.hip) on e4m3: a wavefront multiplies 128 weight rows (FC1:
+// 64 up + the matching 64 gate rows; FC2: 128 output columns) by 32 activation rows over its part of K
+// (L = K / 128 scale blocks of one 128-byte line: part q of kParts takes lines q L / kParts ..
+// (q + 1) L / kParts - 1), and the parts' sums meet in LDS, added in part order. A workgroup holds
+// kGroups runs of 128 weight rows. FC1: two parts, two runs - 128 gated columns, one whole scale group,
+// so with out_codes it also writes the gated rows as FC2's operand. FC2: four parts where they divide
+// the lines (235B: 12), else two parts and two runs (30B: 6 lines, three a part).
+//
+// Bound by HBM (30B T=128 FC1 64 us, 6.3 TB/s). Against the stream kernel (16 or 32 rows a pass, every
+// wavefront loading all the rows): 30B T=128 FC1 73 -> 64 us, FC2 39 -> 35; T=200 80 -> 69, 43.5 ->
+// 38.5; T=300 105 -> 77, 53 -> 47, with Zipf(1.1) routing 283 -> 81, 171 -> 52; 235B T=200 297 -> 255,
+// 156 -> 144. FC1 as eight wavefronts of four parts, one workgroup per CU: T=200 74.
+constexpr int kWideRows = 32;  // rows of a pass
+
+template <bool kGated, int kParts, int kGroups, bool kQuantOut>
+__global__ void __launch_bounds__(kParts * kGroups * kWave) __attribute__((amdgpu_waves_per_eu(2)))
+wide_fp8_kernel(GroupedFp8Params p) {
+  static_assert(!kQuantOut || (kGated && kGroups == 2), "e4m3 out: 128 gated columns");
+  constexpr int kWaves = kParts * kGroups, kThreads = kWaves * kWave;
+  constexpr int kBlocks = kWideRows / 16;
+  constexpr int kColumns = kGated ? 64 : 128;  // output columns of a run
+  __shared__ u32x4 regroup[kWaves][8 * 64];
+  __shared__ int32_t route_list[kExpertRoutes];
+  __shared__ int32_t wave_count[kWaves + 1];
+  __shared__ uint16_t gated_tile[kQuantOut ? 16 * 128 : 1];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int part = wave % kParts;
+  const int lane = lane_id();
+  const int r16 = lane & 15;
+  const int g = lane >> 4;
+  const int64_t live = p.live_tokens != nullptr ? static_cast<int64_t>(p.live_tokens[0]) * p.top : p.routes;
+  const ColumnWork work =
+      column_work<kThreads, kWideRows>(p, live, static_cast<int>(p.out_width / (kColumns * kGroups)), route_list);
+  if (work.expert < 0) return;
+  const int expert = __builtin_amdgcn_readfirstlane(work.expert);
+  const int64_t slice_column = static_cast<int64_t>(work.slice) * (kColumns * kGroups);
+  const int64_t column = slice_column + wave / kParts * kColumns;
+  // Row r (0..127) of the run: FC1 up row column + r, or gate row I + column + r - 64; FC2 output
+  // column `column` + r. Line l of half h: rows 64 h + 8 i + lane / 8, chunk lane % 8.
+  auto weight_row = [&](int r) -> int64_t {
+    if constexpr (kGated) return r < 64 ? column + r : p.out_width + column + (r - 64);
+    else return column + r;
+  };
+  const int lines = static_cast<int>(p.K / 128);
+  const int line_first = part * lines / kParts;
+  const int line_count = (part + 1) * lines / kParts - line_first;
+  const uint32_t row_bytes = static_cast<uint32_t>(p.K);
+  const BufferBase weights = buffer_base(p.weights + expert * p.n_total * p.K, static_cast<uint32_t>(p.n_total) * row_bytes);
+  uint32_t half_off[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    half_off[h] = static_cast<uint32_t>(weight_row(64 * h + lane / 8)) * row_bytes + line_first * 128 + (lane & 7) * 16;
+  struct Half {
+    u32x4 lines[8];
+  };
+  auto load_half = [&](Half &st, int line, int h) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      st.lines[i] = buffer_load16<true>(weights, half_off[h], static_cast<uint32_t>(line) * 128 + i * 8 * row_bytes);
+  };
+  Half even, odd;
+  const FirstRouteIds first_ids = load_first_route_ids<kWaves>(p.ids, p.routes);
+  load_half(even, 0, 0);  // no dependence on the routes: out before the scan (after the ids it reads)
+  // The halves' weight scales: lane l holds line l's of this part (at most 64 lines), read into a
+  // scalar per line.
+  int sw_lanes[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    sw_lanes[h] = __float_as_int(p.weight_scales[(expert * (p.n_total / 128) + weight_row(64 * h) / 128) * lines + line_first +
+                                                 (lane < line_count ? lane : 0)]);
+  const int rows = list_expert_routes<kWaves>(p.ids, p.routes, live, static_cast<int32_t>(expert + p.local_offset),
+                                              route_list, wave_count, &first_ids);
+  if (rows == 0) return;
+  auto listed = [&](int m) -> int64_t { return listed_route<kWaves>(route_list, wave_count, p.routes, m); };
+  const BufferBase act = buffer_base(p.act, 0xffffffffu);
+  const BufferBase act_scales = buffer_base(p.act_scales, 0xffffffffu);
+  const int row_end = min(rows, work.row_last);
+
+  for (int pass = work.row_first; pass < row_end; pass += kWideRows) {
+    uint32_t a_off[kBlocks], s_off[kBlocks];
+#pragma unroll
+    for (int mb = 0; mb < kBlocks; ++mb) {
+      const int m = pass + 16 * mb + r16;
+      int64_t source = 0;  // rows past the expert's routes read row 0 (never stored)
+      if (m < rows) source = kGated ? listed(m) / p.top : listed(m);
+      a_off[mb] = static_cast<uint32_t>(source * p.K + line_first * 128 + g * 16);
+      s_off[mb] = static_cast<uint32_t>((source * lines + line_first) * 4);
+    }
+    floatx4 acc[8][kBlocks];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb) acc[j][mb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    struct Acts {
+      u32x4 lo[kBlocks], hi[kBlocks];  // this lane's 32 K bytes of the line
+      float scale[kBlocks];
+    };
+    Acts xa, xb;
+    auto load_x = [&](Acts &into, int line) {
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb) {
+        into.lo[mb] = buffer_load16<false>(act, a_off[mb], static_cast<uint32_t>(line) * 128);
+        into.hi[mb] = buffer_load16<false>(act, a_off[mb], static_cast<uint32_t>(line) * 128 + 64);
+        into.scale[mb] = buffer_load_f32(act_scales, s_off[mb], static_cast<uint32_t>(line) * 4);
+      }
+    };
+    auto joined = [](const u32x4 &lo, const u32x4 &hi) {
+      return intx8{static_cast<int>(lo[0]), static_cast<int>(lo[1]), static_cast<int>(lo[2]), static_cast<int>(lo[3]),
+                   static_cast<int>(hi[0]), static_cast<int>(hi[1]), static_cast<int>(hi[2]), static_cast<int>(hi[3])};
+    };
+    auto compute = [&](const Half &st, int h, int line, const Acts &xs) {
+      {
+        const int row = lane >> 3, piece = lane & 7;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) regroup[wave][i * 64 + row * 8 + (piece ^ row)] = st.lines[i];
+      }
+      const float sw = __int_as_float(__builtin_amdgcn_readlane(sw_lanes[h], line));
+      float scale[kBlocks];
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb) scale[mb] = sw * xs.scale[mb];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 2 * j + (r16 >> 3), rr = r16 & 7;
+        const intx8 w = joined(regroup[wave][i * 64 + rr * 8 + (g ^ rr)], regroup[wave][i * 64 + rr * 8 + ((g + 4) ^ rr)]);
+#pragma unroll
+        for (int mb = 0; mb < kBlocks; ++mb) {
+          const floatx4 block = mfma_16x16x128_fp8(w, joined(xs.lo[mb], xs.hi[mb]), floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[4 * h + j][mb][e] = __builtin_fmaf(block[e], scale[mb], acc[4 * h + j][mb][e]);
+        }
+      }
+    };
+    if (pass > work.row_first) load_half(even, 0, 0);
+    load_x(xa, 0);
+    load_half(odd, 0, 1);
+    // A line that has a next one: its halves' buffers are filled with the next line's as soon as
+    // they are consumed, all unconditionally, so each wait counts exactly the loads still in flight.
+    auto line = [&](int l, const Acts &now, Acts &next) {
+      load_x(next, l + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(even, 0, l, now);
+      __builtin_amdgcn_sched_barrier(0);
+      load_half(even, l + 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(odd, 1, l, now);
+      __builtin_amdgcn_sched_barrier(0);
+      load_half(odd, l + 1, 1);
+    };
+    auto last_line = [&](int l, const Acts &now) {
+      compute(even, 0, l, now);
+      compute(odd, 1, l, now);
+    };
+    int l = 0;
+    for (; l + 2 < line_count; l += 2) {
+      line(l, xa, xb);
+      line(l + 1, xb, xa);
+    }
+    if (l + 1 < line_count) {
+      line(l, xa, xb);
+      last_line(l + 1, xb);
+    } else {
+      last_line(l, xa);
+    }
+
+    // The parts' sums of a run, added in part order, one row block at a time, through the regroup
+    // buffers (8 x 64 floatx4 each), which are no longer read. Part q stores sets q kSets .. of the
+    // run (FC1: of its up rows, gated by the same sets of its gate rows).
+    constexpr int kSets = (kGated ? 4 : 8) / kParts;
+    auto partial = [&](int w, int j) -> floatx4 & { return reinterpret_cast<floatx4 *>(regroup[w])[j * kWave + lane]; };
+    auto total = [&](int j) {
+      floatx4 sum = partial(wave - part, j);
+#pragma unroll
+      for (int w = 1; w < kParts; ++w) sum += partial(wave - part + w, j);
+      return sum;
+    };
+#pragma unroll
+    for (int mb = 0; mb < kBlocks; ++mb) {
+      if (pass + 16 * mb >= rows) break;  // (uniform)
+      if (mb > 0) __syncthreads();        // the block before is summed (and its tile quantised)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) partial(wave, j) = acc[j][mb];
+      __syncthreads();
+      const int m = pass + 16 * mb + r16;
+      uint16_t *row = p.out + (m < rows ? listed(m) : 0) * p.out_width + column + 4 * g;
+#pragma unroll
+      for (int s = 0; s < kSets; ++s) {
+        const int j = part * kSets + s;
+        floatx4 v = total(j);
+        if constexpr (kGated) {
+          const floatx4 gated = total(j + 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = gate(gated[e], p.activation) * v[e];
+        }
+        if (m >= rows) continue;
+        store_bf16x4(row + j * 16, v);
+        if constexpr (kQuantOut) store_bf16x4(gated_tile + r16 * 128 + wave / kParts * 64 + j * 16 + 4 * g, v);
+      }
+      if constexpr (kQuantOut) {
+        // The block's rows x the workgroup's 128 columns (one scale group), 16 lanes a row.
+        __syncthreads();
+        const int t = static_cast<int>(threadIdx.x);
+        const int r = t / 16, mr = pass + 16 * mb + r;
+        if (r < 16 && mr < rows) {
+          const int64_t route = listed(mr);
+          quantize_bf16_group(gated_tile + r * 128, p.out_codes + route * p.out_width + slice_column,
+                              p.out_code_scales + route * (p.out_width / 128) + slice_column / 128, t & 15);
+        }
+      }
+    }
+    __syncthreads();  // the next pass's lines overwrite the partial sums
+  }
+}
+
 /// Prefill-shaped: 128 x 128 tiles, one 128-deep scale block per LDS stage (16 KB per operand).
 constexpr int kStageChunks = 128 * 8;  // 16-byte chunks: 128 rows x 128 bytes
 
@@ -623,6 +838,19 @@ bool expert_stream_fp8_fc1_quantizes(int64_t routes, int64_t local_experts, int6
   return served * (out_width / 64) >= kSplitBelow && out_width % 128 == 0;
 }
 
+/// Whether the wide kernel takes the unsplit expert-major product (p.experts, the router's): above two
+/// rows per expert on average, and FC1 from 4096 channels at any (235B T=4 68 -> 62 us, T=16 186 -> 171);
+/// below, the stream kernel's workgroups need no exchange of partial sums (30B T=32 FC1 59.0 us against
+/// 59.8; FC2 T=5 12.6 against 14.8, 235B T=16 93 against 96). A part holds at most 64 lines' scales; byte
+/// offsets of an expert's weights and of the activations stay below 2^32.
+bool wide_fp8_fits(const GroupedFp8Params &p, bool gated) {
+  constexpr int64_t kOffsetRange = int64_t{1} << 32;
+  const int64_t lines = p.K / 128;
+  const bool rows = p.routes > 2 * p.experts || (gated && lines >= 32);
+  return rows && (gated ? p.out_codes != nullptr : lines % 4 == 0 || p.out_width % 256 == 0) && lines >= 2 &&
+         lines <= 128 && p.n_total * p.K < kOffsetRange && p.routes * p.K < kOffsetRange;
+}
+
 void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, int64_t local_experts, hipStream_t stream) {
   GroupedFp8Params p = params;
   p.local_experts = local_experts;
@@ -644,20 +872,26 @@ void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, int64_
     else hipLaunchKernelGGL((stream_fp8_kernel<false, true, 2, true>), grid, dim3(kThreads), 0, stream, p);
     return;
   }
+  if (wide_fp8_fits(p, gated)) {
+    p.columns = static_cast<int32_t>(columns);
+    p.extra_columns = extra_columns(p.routes, p.top, local_experts, p.compact != 0, kWideRows);
+    const bool four = p.K / 128 % 4 == 0;
+    const int64_t runs = gated || four ? p.out_width / 128 : p.out_width / 256;
+    const dim3 grid(static_cast<uint32_t>((p.columns + p.extra_columns) * runs));
+    if (gated) hipLaunchKernelGGL((wide_fp8_kernel<true, 2, 2, true>), grid, dim3(kThreads), 0, stream, p);
+    else if (four) hipLaunchKernelGGL((wide_fp8_kernel<false, 4, 1, false>), grid, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((wide_fp8_kernel<false, 2, 2, false>), grid, dim3(kThreads), 0, stream, p);
+    return;
+  }
   if (gated && p.out_codes != nullptr) {
     // The gated rows also as FC2's operand: eight-wave workgroups of 128 gated columns.
     const dim3 grid(static_cast<uint32_t>(columns), static_cast<uint32_t>(p.out_width / 128));
-    if (one_pass)
-      hipLaunchKernelGGL((stream_fp8_kernel<true, false, 1, true, 1, 8, true>), grid, dim3(8 * kWave), 0, stream, p);
-    else
-      hipLaunchKernelGGL((stream_fp8_kernel<true, false, 2, true, 1, 8, true>), grid, dim3(8 * kWave), 0, stream, p);
+    hipLaunchKernelGGL((stream_fp8_kernel<true, false, 1, true, 1, 8, true>), grid, dim3(8 * kWave), 0, stream, p);
     return;
   }
   const dim3 grid(static_cast<uint32_t>(columns), static_cast<uint32_t>(slices));
-  if (gated && one_pass) hipLaunchKernelGGL((stream_fp8_kernel<true, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
-  else if (gated) hipLaunchKernelGGL((stream_fp8_kernel<true, false, 2, true>), grid, dim3(kThreads), 0, stream, p);
-  else if (one_pass) hipLaunchKernelGGL((stream_fp8_kernel<false, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
-  else hipLaunchKernelGGL((stream_fp8_kernel<false, false, 2, true>), grid, dim3(kThreads), 0, stream, p);
+  if (gated) hipLaunchKernelGGL((stream_fp8_kernel<true, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
+  else hipLaunchKernelGGL((stream_fp8_kernel<false, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
 }
 
 }  // namespace uniserve

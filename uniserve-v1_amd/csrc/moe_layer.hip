@@ -627,6 +627,7 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
         e.live_tokens = call->live_tokens;
         e.routes = routes;
         e.local_offset = call->local_offset;
+        e.experts = call->experts;
         e.top = call->top;
         e.activation = activation;
         // Where the unsplit kernel serves FC1 it also writes FC2's operand (QUANTIZE_GATED then
