@@ -136,8 +136,15 @@ buffer_load16(BufferBase base, uint32_t lane_offset, uint32_t offset) {
   return __builtin_amdgcn_raw_buffer_load_b128(base, lane_offset, offset, kOnce ? 2 : 0);
 }
 
+__device__ __forceinline__ uint32_t buffer_load_u32(BufferBase base, uint32_t lane_offset, uint32_t offset) {
+  return __builtin_amdgcn_raw_buffer_load_b32(base, lane_offset, offset, 0);
+}
+__device__ __forceinline__ uint2 buffer_load_u32x2(BufferBase base, uint32_t lane_offset, uint32_t offset) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b64(base, lane_offset, offset, 0);
+  return uint2{v[0], v[1]};
+}
 __device__ __forceinline__ float buffer_load_f32(BufferBase base, uint32_t lane_offset, uint32_t offset) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(base, lane_offset, offset, 0));
+  return __uint_as_float(buffer_load_u32(base, lane_offset, offset));
 }
 
 // ---- MFMA operands ------------------------------------------------------------------------------------

@@ -38,6 +38,7 @@ struct ExpertRouting {
   const int32_t *ids;
   const int32_t *live_tokens;
   int64_t routes, top, local_offset, local_experts;
+  int64_t experts;  ///< the router's (routes / experts: the rows an expert expects)
 };
 
 /// With `codes` (and `code_scales`), FC1 also writes the gated rows as FC2's MXFP8 operand (codes

@@ -132,6 +132,8 @@ struct MxParams {
   int64_t local_offset;
   int64_t local_experts;
   int32_t compact;
+  int32_t columns;               ///< wide kernel: workgroup columns (experts, or routes if compact)
+  int32_t extra_columns;         ///< wide kernel: columns past those, for rows past an expert's first pass
   // FC1 on the tiled kernel only, or null: the gated rows are written as MXFP8 codes
   // [permuted_rows, out_width] with their E8M0 bytes stage-major by permuted row
   // ([out_width / 128, code_scale_rows, 4]) instead of bf16 rows - FC2's operand.
@@ -452,6 +454,230 @@ __global__ void __launch_bounds__(kThreads) stream_mx_kernel(MxParams p) {
       __syncthreads();
     }
   }
+  }
+}
+
+// ---- the wide kernel (decode and continuous batches, expert-major) ------------------------------------------
+//
+// The bf16 wide kernel's form (grouped_gemm.hip) on MXFP4: a wavefront multiplies 128 weight rows (FC1:
+// 64 up + the matching 64 gate rows; FC2: 128 output columns) by 32 activation rows over its part of K
+// (L = K / 256 lines of 128 bytes of pairs, two MFMAs each), and the parts' sums meet in LDS, added in
+// part order. A workgroup holds kGroups runs of 128 weight rows. FC1: two parts, two runs; with
+// out_codes its 128 gated columns leave as FC2's MXFP8 operand too. FC2: two parts and two runs where
+// the lines are even (235B: 6), else each wavefront a run of its own over all of K (30B: 3 lines). A
+// half's weight scales, one word per row and 128 K elements, come a row per lane and reach the lanes
+// that multiply by them through LDS beside the lines.
+//
+// Bound by HBM (235B T=64 FC1 125 us, 6.4 TB/s). Against the stream kernel (16 rows a pass, every
+// wavefront loading all the rows): 30B T=128 FC1 48 -> 42 us, FC2 31 -> 21; T=200 65 -> 46, 41.5 -> 24;
+// T=300 with Zipf(1.1) routing 336 -> 56, 351 -> 39; 235B T=23 114 -> 106, 62.5 -> 58; T=200 234 -> 149,
+// 132 -> 87.
+constexpr int kWideRows = 32;  // rows of a pass
+
+template <bool kGated, int kParts, int kGroups, bool kQuantOut>
+__global__ void __launch_bounds__(kParts * kGroups * kWave) __attribute__((amdgpu_waves_per_eu(2)))
+wide_mx_kernel(MxParams p) {
+  static_assert(kParts * kGroups * kWave == kThreads, "four wavefronts");
+  constexpr int kWaves = kParts * kGroups;
+  constexpr int kBlocks = kWideRows / 16;
+  constexpr int kColumns = kGated ? 64 : 128;  // output columns of a run
+  constexpr int kTileColumns = kColumns * kGroups;
+  __shared__ u32x4 regroup[kWaves][8 * 64];
+  __shared__ uint32_t scale_words[kWaves][2 * kWave];
+  __shared__ int32_t route_list[kExpertRoutes];
+  __shared__ int32_t wave_count[kWaves + 1];
+  __shared__ uint16_t gated_tile[kQuantOut ? 16 * kTileColumns : 1];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int part = wave % kParts;
+  const int lane = lane_id();
+  const int r16 = lane & 15;
+  const int g = lane >> 4;
+  const int64_t live = p.live_tokens != nullptr ? static_cast<int64_t>(p.live_tokens[0]) * p.top : p.routes;
+  const ColumnWork work = column_work<kThreads, kWideRows>(p, live, static_cast<int>(p.out_width / kTileColumns), route_list);
+  if (work.expert < 0) return;
+  const int expert = __builtin_amdgcn_readfirstlane(work.expert);
+  const int64_t slice_column = static_cast<int64_t>(work.slice) * kTileColumns;
+  const int64_t column = slice_column + wave / kParts * kColumns;
+  // Row r (0..127) of the run: FC1 up row column + r, or gate row I + column + r - 64; FC2 output
+  // column `column` + r. Line l of half h: rows 64 h + 8 i + lane / 8, chunk lane % 8.
+  auto weight_row = [&](int r) -> int64_t {
+    if constexpr (kGated) return r < 64 ? column + r : p.out_width + column + (r - 64);
+    else return column + r;
+  };
+  const int lines = static_cast<int>(p.K / 256);
+  const int line_first = part * lines / kParts;
+  const int line_count = (part + 1) * lines / kParts - line_first;
+  const uint32_t row_bytes = static_cast<uint32_t>(p.K / 2);
+  const BufferBase weights = buffer_base(p.weights + expert * p.n_total * (p.K / 2), static_cast<uint32_t>(p.n_total) * row_bytes);
+  const BufferBase scales = buffer_base(p.weight_scales + expert * p.n_total * (p.K / 32),
+                                        static_cast<uint32_t>(p.n_total * (p.K / 32)));
+  const uint32_t ws_stage = static_cast<uint32_t>(p.ws_stage);
+  uint32_t half_off[2], ws_off[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    half_off[h] = static_cast<uint32_t>(weight_row(64 * h + lane / 8)) * row_bytes + line_first * 128 + (lane & 7) * 16;
+    ws_off[h] = static_cast<uint32_t>(weight_row(64 * h + lane)) * static_cast<uint32_t>(p.ws_row) + 2 * line_first * ws_stage;
+  }
+  struct Half {
+    u32x4 lines[8];
+    uint32_t scales[2];
+  };
+  auto load_half = [&](Half &st, int line, int h) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      st.lines[i] = buffer_load16<true>(weights, half_off[h], static_cast<uint32_t>(line) * 128 + i * 8 * row_bytes);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) st.scales[s] = buffer_load_u32(scales, ws_off[h], (2 * static_cast<uint32_t>(line) + s) * ws_stage);
+  };
+  Half even, odd;
+  const FirstRouteIds first_ids = load_first_route_ids<kWaves>(p.ids, p.routes);
+  load_half(even, 0, 0);  // no dependence on the routes: out before the scan (after the ids it reads)
+  const int rows = list_expert_routes<kWaves>(p.ids, p.routes, live, static_cast<int32_t>(expert + p.local_offset),
+                                              route_list, wave_count, &first_ids);
+  if (rows == 0) return;
+  auto listed = [&](int m) -> int64_t { return listed_route<kWaves>(route_list, wave_count, p.routes, m); };
+  const BufferBase act = buffer_base(p.act, 0xffffffffu);
+  const BufferBase act_scales = buffer_base(p.act_scales, 0xffffffffu);
+  const int row_end = min(rows, work.row_last);
+
+  for (int pass = work.row_first; pass < row_end; pass += kWideRows) {
+    uint32_t a_off[kBlocks], s_off[kBlocks];
+#pragma unroll
+    for (int mb = 0; mb < kBlocks; ++mb) {
+      const int m = pass + 16 * mb + r16;
+      int64_t source = 0;  // rows past the expert's routes read row 0 (never stored)
+      if (m < rows) source = kGated ? listed(m) / p.top : listed(m);
+      a_off[mb] = static_cast<uint32_t>(source * p.K + line_first * 256 + g * 16);
+      s_off[mb] = static_cast<uint32_t>(source * p.as_row + line_first * 8);  // (row-major scales)
+    }
+    floatx4 acc[8][kBlocks];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb) acc[j][mb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    struct Acts {
+      u32x4 lo[kBlocks][2], hi[kBlocks][2];  // this lane's 32 K bytes of each 128 of the line
+      uint2 scale[kBlocks];
+    };
+    Acts x;
+    auto load_x = [&](Acts &into, int line) {
+#pragma unroll
+      for (int mb = 0; mb < kBlocks; ++mb) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          into.lo[mb][s] = buffer_load16<false>(act, a_off[mb], static_cast<uint32_t>(line) * 256 + 128 * s);
+          into.hi[mb][s] = buffer_load16<false>(act, a_off[mb], static_cast<uint32_t>(line) * 256 + 128 * s + 64);
+        }
+        into.scale[mb] = buffer_load_u32x2(act_scales, s_off[mb], static_cast<uint32_t>(line) * 8);
+      }
+    };
+    auto joined = [](const u32x4 &lo, const u32x4 &hi) {
+      return intx8{static_cast<int>(lo[0]), static_cast<int>(lo[1]), static_cast<int>(lo[2]), static_cast<int>(lo[3]),
+                   static_cast<int>(hi[0]), static_cast<int>(hi[1]), static_cast<int>(hi[2]), static_cast<int>(hi[3])};
+    };
+    auto compute = [&](const Half &st, int h, const Acts &xs) {
+      {
+        const int row = lane >> 3, piece = lane & 7;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) regroup[wave][i * 64 + row * 8 + (piece ^ row)] = st.lines[i];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) scale_words[wave][s * kWave + lane] = st.scales[s];
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        uint32_t sx[kBlocks];
+#pragma unroll
+        for (int mb = 0; mb < kBlocks; ++mb) sx[mb] = ((s == 0 ? xs.scale[mb].x : xs.scale[mb].y) >> (8 * g)) & 0xffu;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int rr = r16 & 7, q = 4 * s + g;
+          const u32x4 w = regroup[wave][(2 * j + (r16 >> 3)) * 64 + rr * 8 + (q ^ rr)];
+          const uint32_t sw = (scale_words[wave][s * kWave + 16 * j + r16] >> (8 * g)) & 0xffu;
+#pragma unroll
+          for (int mb = 0; mb < kBlocks; ++mb)
+            acc[4 * h + j][mb] = mfma_mx(w, joined(xs.lo[mb][s], xs.hi[mb][s]), sw, sx[mb], acc[4 * h + j][mb]);
+        }
+      }
+    };
+    if (pass > work.row_first) load_half(even, 0, 0);
+    load_x(x, 0);
+    load_half(odd, 0, 1);
+    // The halves' buffers and the activations are refilled with the next line's as soon as they are
+    // consumed, unconditionally but for the last line's, so each wait counts exactly the loads still in
+    // flight. (A second activation buffer spills.)
+    for (int l = 0; l + 1 < line_count; ++l) {
+      compute(even, 0, x);
+      __builtin_amdgcn_sched_barrier(0);
+      load_half(even, l + 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(odd, 1, x);
+      __builtin_amdgcn_sched_barrier(0);
+      load_x(x, l + 1);
+      load_half(odd, l + 1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    compute(even, 0, x);
+    compute(odd, 1, x);
+
+    // The parts' sums of a run, added in part order, one row block at a time, through the regroup
+    // buffers (8 x 64 floatx4 each), which are no longer read. Part q stores sets q kSets .. of the
+    // run (FC1: of its up rows, gated by the same sets of its gate rows).
+    constexpr int kSets = (kGated ? 4 : 8) / kParts;
+    auto partial = [&](int w, int j) -> floatx4 & { return reinterpret_cast<floatx4 *>(regroup[w])[j * kWave + lane]; };
+#pragma unroll
+    for (int mb = 0; mb < kBlocks; ++mb) {
+      if (pass + 16 * mb >= rows) break;  // (uniform)
+      auto total = [&](int j) {
+        if constexpr (kParts == 1) return acc[j][mb];
+        floatx4 sum = partial(wave - part, j);
+#pragma unroll
+        for (int w = 1; w < kParts; ++w) sum += partial(wave - part + w, j);
+        return sum;
+      };
+      if constexpr (kParts > 1) {
+        if (mb > 0) __syncthreads();  // the block before is summed (and its tile quantised)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) partial(wave, j) = acc[j][mb];
+        __syncthreads();
+      }
+      const int m = pass + 16 * mb + r16;
+      uint16_t *row = p.out + (m < rows ? listed(m) : 0) * p.out_width + column + 4 * g;
+#pragma unroll
+      for (int s = 0; s < kSets; ++s) {
+        const int j = part * kSets + s;
+        floatx4 v = total(j);
+        if constexpr (kGated) {
+          const floatx4 gated = total(j + 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = gate(gated[e], p.activation) * v[e];
+        }
+        if (m >= rows) continue;
+        store_bf16x4(row + j * 16, v);
+        if constexpr (kQuantOut) store_bf16x4(gated_tile + r16 * kTileColumns + wave / kParts * 64 + j * 16 + 4 * g, v);
+      }
+      if constexpr (kQuantOut) {
+        // The block's rows x the workgroup's 32-column blocks, four lanes a block.
+        static_assert(kParts > 1 && 16 * (kTileColumns / 32) * 4 == kThreads, "one block per four lanes");
+        __syncthreads();
+        const int t = static_cast<int>(threadIdx.x);
+        const int r = t / (kTileColumns / 8), block = t / 4 % (kTileColumns / 32), sub = t & 3;
+        const int mr = pass + 16 * mb + r;
+        if (mr < rows) {
+          const u32x4 bits = *reinterpret_cast<const u32x4 *>(gated_tile + r * kTileColumns + block * 32 + sub * 8);
+          float v[8];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            v[2 * j] = __uint_as_float(bits[j] << 16);
+            v[2 * j + 1] = __uint_as_float(bits[j] & 0xffff0000u);
+          }
+          const int64_t route = listed(mr);
+          const int64_t at = slice_column + block * 32;
+          const uint32_t scale = mxfp8_eight(v, p.out_codes + route * p.out_width + at + sub * 8);
+          if (sub == 0) p.out_code_scales[route * (p.out_width / 32) + at / 32] = static_cast<uint8_t>(scale);
+        }
+      }
+    }
+    if constexpr (kParts > 1) __syncthreads();  // the next pass's lines overwrite the partial sums
   }
 }
 
@@ -947,6 +1173,18 @@ constexpr int kFc2Run = 4;
 /// 235B T=1 FC2 14.2 -> 11.6 us by events (four: 15.9, eight: 23.2).
 constexpr int kSplitFc2Run = 2;
 
+/// Whether the wide kernel takes the unsplit expert-major product: FC2 always (30B T=5 13.7 -> 10.5 us,
+/// T=64 21.7 -> 19.1), FC1 above two rows per expert on average, or one from 4096 channels (30B T=32 33.9
+/// us on the stream kernel against 36.7; 235B T=4 32.8 against 37.3, T=16 108.9 against 97.4).
+bool wide_mx_fits(const MxParams &p, bool gated, int64_t experts) {
+  const int64_t lines = p.K / 256;
+  constexpr int64_t kOffsetRange = int64_t{1} << 32;  // an expert's weights and the activations
+  if (lines < 2 || p.n_total * (p.K / 2) >= kOffsetRange || p.routes * p.K >= kOffsetRange) return false;
+  if (!gated) return p.out_width % (lines % 2 == 0 ? 256 : 512) == 0;
+  return p.out_codes != nullptr && p.out_width % 128 == 0 &&
+         (p.routes > 2 * experts || (p.K >= 4096 && p.routes >= experts));
+}
+
 void launch_expert_mx(MxParams p, bool gated, const ExpertRouting &r, hipStream_t stream) {
   p.ids = r.ids;
   p.live_tokens = r.live_tokens;
@@ -967,6 +1205,17 @@ void launch_expert_mx(MxParams p, bool gated, const ExpertRouting &r, hipStream_
     } else {
       hipLaunchKernelGGL((stream_mx_kernel<false, true, true>), grid, dim3(kThreads), 0, stream, p);
     }
+    return;
+  }
+  const bool two = p.K / 256 % 2 == 0;
+  if (wide_mx_fits(p, gated, r.experts)) {
+    p.columns = static_cast<int32_t>(columns);
+    p.extra_columns = extra_columns(p.routes, p.top, p.local_experts, p.compact != 0, kWideRows);
+    const int64_t runs = p.out_width / (gated ? 128 : two ? 256 : 512);
+    const dim3 grid(static_cast<uint32_t>((p.columns + p.extra_columns) * runs));
+    if (gated) hipLaunchKernelGGL((wide_mx_kernel<true, 2, 2, true>), grid, dim3(kThreads), 0, stream, p);
+    else if (two) hipLaunchKernelGGL((wide_mx_kernel<false, 2, 2, false>), grid, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((wide_mx_kernel<false, 1, 4, false>), grid, dim3(kThreads), 0, stream, p);
     return;
   }
   if (gated && p.out_codes != nullptr) {

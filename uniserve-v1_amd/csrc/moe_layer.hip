@@ -519,7 +519,7 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
 
     // 4-5. The two products.
     if (mx) {
-      const ExpertRouting routing{ids, call->live_tokens, routes, call->top, call->local_offset, local_experts};
+      const ExpertRouting routing{ids, call->live_tokens, routes, call->top, call->local_offset, local_experts, call->experts};
       if (int32_t status = run_mx_products(call, v, ws, want, stream, by_expert ? &routing : nullptr,
                                                  front_quantizes || prefill_quantizes,
                                                  prefill_quantizes && v.route_scales && !sort_scatters))
