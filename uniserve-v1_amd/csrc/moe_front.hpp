@@ -65,7 +65,8 @@ bool split_front_fits(int64_t tokens, int64_t experts, int64_t hidden, int64_t t
 void launch_split_front(const FrontParams &p, hipStream_t stream);
 
 /// The front end at prefill sizes (front_prefill.hip): router scores, topk and (with `codes`) the
-/// hidden rows' quantisation in one launch, one workgroup per 32 tokens.
+/// hidden rows' quantisation in one launch, one workgroup per 32 tokens, or (up to 4096 tokens) in two,
+/// the experts of each 32 tokens split over workgroups.
 struct PrefillFrontParams {
   const uint16_t *x;        ///< [tokens, hidden] bf16
   const uint16_t *w;        ///< [experts, hidden] bf16 router
@@ -88,11 +89,17 @@ struct PrefillFrontParams {
   /// the sort's count of the workgroup's 32 tokens (kFrontChunkTokens).
   int32_t *chunk_counts;
   int32_t local_offset, local_experts;
+  /// Or null (split launches only): [tokens, top], each visible route's own expanded index, -1 elsewhere
+  /// (for products that find their routes themselves), with local_offset and local_experts set.
+  int32_t *expanded_to_permuted;
 };
 
 /// Whether one launch serves these extents: at most 128 experts picking at most 32, whole
 /// 128-channel stages.
 bool prefill_front_fits(int64_t tokens, int64_t experts, int64_t hidden, int64_t top);
+
+/// Workgroups the launch shares each 32 tokens out to (1: the single-launch kernel).
+int prefill_front_split(int64_t tokens);
 
 void launch_prefill_front(const PrefillFrontParams &p, hipStream_t stream);
 

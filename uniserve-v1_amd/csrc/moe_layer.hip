@@ -33,6 +33,9 @@ namespace {
 
 constexpr int64_t kTile = 128;
 constexpr int64_t kAlign = 256;
+// Tokens up to which the expert-split front end serves, and between which the one with a workgroup per
+// token does (at most one per CU).
+constexpr int64_t kSplitFrontMost = 8, kTokenFrontLeast = 32, kTokenFrontMost = 256;
 
 int64_t aligned(int64_t bytes) { return (bytes + kAlign - 1) / kAlign * kAlign; }
 
@@ -351,6 +354,13 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
 
     // e4m3 and MXFP4 at those sizes: the front end also quantises the hidden rows (QUANTIZE_HIDDEN
     // then launches nothing).
+    // Layers without a sort past the smallest batches: the prefill front end's split launches, except
+    // where a workgroup per token has a CU to itself and rows short enough (30B T=64 11.5 us against 11.6;
+    // past one token per CU, T=301, 21.7 against 12.6; 235B T=64 17.7 against 14.9, T=16 16.1 against 14.5).
+    const bool chunk_front = by_expert && call->tokens > kSplitFrontMost &&
+                             (call->tokens < kTokenFrontLeast || call->tokens > kTokenFrontMost || call->hidden_size >= 4096) &&
+                             prefill_front_fits(call->tokens, call->experts, call->hidden_size, call->top) &&
+                             prefill_front_split(call->tokens) > 1;
     const bool front_quantizes = front && (fp8 || mx) && !v.route_scales && call->hidden_size % 128 == 0;
     // Prefill sizes: router scores, topk and (e4m3, MXFP4) the hidden rows' quantisation in one
     // launch (ROUTER; TOPK launches nothing). The scales come out token-major; where the products
@@ -389,7 +399,35 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
 
     // Decode sizes: router, topk and sort in one launch (at the ROUTER step; TOPK and SORT launch
     // nothing).
-    if (front) {
+    if (chunk_front) {
+      if (want(UNISERVE_MOE_LAYER_ROUTER)) {
+        PrefillFrontParams pp{};
+        pp.x = static_cast<const uint16_t *>(call->hidden);
+        pp.w = static_cast<const uint16_t *>(call->router);
+        pp.bias = call->router_bias;
+        pp.scores = static_cast<uint16_t *>(at(v.scores));
+        pp.tokens = call->tokens;
+        pp.experts = call->experts;
+        pp.hidden = call->hidden_size;
+        pp.top = static_cast<int32_t>(call->top);
+        pp.renormalize = call->renormalize ? 1 : 0;
+        pp.map = call->map;
+        pp.live = call->live_tokens;
+        pp.load = reinterpret_cast<unsigned long long *>(call->load);
+        pp.ids = ids;
+        pp.weights = weights;
+        pp.local_offset = static_cast<int32_t>(call->local_offset);
+        pp.local_experts = static_cast<int32_t>(local_experts);
+        pp.expanded_to_permuted = e2p;
+        if (front_quantizes) {
+          pp.codes = static_cast<uint8_t *>(at(v.hidden_q));
+          if (mx) pp.mx_scales = static_cast<uint8_t *>(at(v.hidden_s));
+          else pp.scales = static_cast<float *>(at(v.hidden_s));
+        }
+        launch_prefill_front(pp, s);
+        if (int32_t status = launched(call, "router and topk")) return status;
+      }
+    } else if (front) {
       if (want(UNISERVE_MOE_LAYER_ROUTER)) {
         FrontParams fp{};
         fp.x = static_cast<const uint16_t *>(call->hidden);
@@ -749,9 +787,9 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
     combine.layout = by_expert ? UNISERVE_UNPERMUTE_LAYOUT_EXPANDED : UNISERVE_UNPERMUTE_LAYOUT_PERMUTED;
     // After the fused front end the combine also checks that the front end's counters came back to
     // zero (they do unless they were not zero before it: a workspace whose head was not cleared).
-    uint32_t *ticket = front ? static_cast<uint32_t *>(at(v.ticket)) : nullptr;
+    uint32_t *ticket = front && !chunk_front ? static_cast<uint32_t *>(at(v.ticket)) : nullptr;
     if (want(UNISERVE_MOE_LAYER_UNPERMUTE) &&
-        moe_unpermute_checked(&combine, ticket, front ? front_ticket_words(call->tokens) : 0, stream) != 0)
+        moe_unpermute_checked(&combine, ticket, ticket != nullptr ? front_ticket_words(call->tokens) : 0, stream) != 0)
       return forward_error(call, "moe_unpermute", combine);
     return 0;
   });
