@@ -624,14 +624,14 @@ constexpr int64_t kStreamRowsPerExpert = 24;
 
 /// FC2 by expert with at most this many rows per expert on average stays on the stream kernel,
 /// whose workgroups need no exchange of partial sums (30B: T=5 21.1 us against 23.4 on the wide
-/// kernel, T=64 62.0 against 62.5 - with Zipf routing, where some experts have more than 16 rows, 86
+/// kernel, T=40 58.2 against 59.5, T=64 61.8 against 61.8 - with Zipf routing, where some experts have more than 16 rows, 86
 /// against 50 - and T=128 70 against 65).
-constexpr int64_t kWideFc2RowsPerExpert = 2;
+constexpr int64_t kWideFc2RowsPerExpert = 3;
 
 /// FC1 by expert with at most this many rows per expert on average: 16 rows a pass, whose fewer
-/// registers leave three waves per SIMD (30B: T=32 104 us against 107; T=64 117.6 against 118.3, but
-/// 150 against 98 with Zipf routing, where some experts have more rows than that).
-constexpr int64_t kWideOneBlockRowsPerExpert = 2;
+/// registers leave three waves per SIMD (30B: T=32 104 us against 107, T=64 117.5 against 118.3, with
+/// Zipf routing, whose further runs of 16 rows are shared out, 82 against 98).
+constexpr int64_t kWideOneBlockRowsPerExpert = 4;
 
 /// By the sort's tiles: workgroups below which the wide kernel is not worth its exchange.
 constexpr int64_t kWideWorkgroups = 170;
@@ -707,10 +707,11 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
   if (wide_fits(p, e.routes) && (gated || e.routes > kWideFc2RowsPerExpert * e.experts)) {
     // An expert with more rows than one pass takes leaves the rest to workgroups of their own (with
     // one column per expert that may have any: nth_extra_run).
-    p.extra_columns = extra_columns(e.routes, e.top, e.local_experts, p.compact != 0, kWideRows);
+    const bool one_block = gated && e.routes <= kWideOneBlockRowsPerExpert * e.experts;
+    p.extra_columns = extra_columns(e.routes, e.top, e.local_experts, p.compact != 0, one_block ? 16 : kWideRows);
     p.columns = static_cast<int32_t>(grid.x);
     const dim3 wide_grid(static_cast<uint32_t>((p.columns + p.extra_columns) * slices));
-    if (gated && e.routes <= kWideOneBlockRowsPerExpert * e.experts)
+    if (one_block)
       hipLaunchKernelGGL((wide_kernel<true, true, 1>), wide_grid, dim3(kThreads), 0, stream, p);
     else if (gated) hipLaunchKernelGGL((wide_kernel<true, true>), wide_grid, dim3(kThreads), 0, stream, p);
     else hipLaunchKernelGGL((wide_kernel<false, true>), wide_grid, dim3(kThreads), 0, stream, p);

@@ -839,14 +839,15 @@ bool expert_stream_fp8_fc1_quantizes(int64_t routes, int64_t local_experts, int6
 }
 
 /// Whether the wide kernel takes the unsplit expert-major product (p.experts, the router's): above two
-/// rows per expert on average, and FC1 from 4096 channels at any (235B T=4 68 -> 62 us, T=16 186 -> 171);
-/// below, the stream kernel's workgroups need no exchange of partial sums (30B T=32 FC1 59.0 us against
-/// 59.8; FC2 T=5 12.6 against 14.8, 235B T=16 93 against 96). A part holds at most 64 lines' scales; byte
+/// (FC1: three) rows per expert on average, and FC1 from 4096 channels at any (235B T=4 68 -> 62 us, T=16
+/// 186 -> 171); below, the stream kernel's workgroups need no exchange of partial sums (30B T=32 FC1 59.0 us
+/// against 59.8, T=64 63.4 against 63.7, with Zipf routing 130 against 67; FC2 T=5 12.6 against 14.8, 235B
+/// T=16 93 against 96). A part holds at most 64 lines' scales; byte
 /// offsets of an expert's weights and of the activations stay below 2^32.
 bool wide_fp8_fits(const GroupedFp8Params &p, bool gated) {
   constexpr int64_t kOffsetRange = int64_t{1} << 32;
   const int64_t lines = p.K / 128;
-  const bool rows = p.routes > 2 * p.experts || (gated && lines >= 32);
+  const bool rows = p.routes > (gated ? 3 : 2) * p.experts || (gated && lines >= 32);
   return rows && (gated ? p.out_codes != nullptr : lines % 4 == 0 || p.out_width % 256 == 0) && lines >= 2 &&
          lines <= 128 && p.n_total * p.K < kOffsetRange && p.routes * p.K < kOffsetRange;
 }

@@ -1174,15 +1174,15 @@ constexpr int kFc2Run = 4;
 constexpr int kSplitFc2Run = 2;
 
 /// Whether the wide kernel takes the unsplit expert-major product: FC2 always (30B T=5 13.7 -> 10.5 us,
-/// T=64 21.7 -> 19.1), FC1 above two rows per expert on average, or one from 4096 channels (30B T=32 33.9
-/// us on the stream kernel against 36.7; 235B T=4 32.8 against 37.3, T=16 108.9 against 97.4).
+/// T=64 21.7 -> 19.1), FC1 above three rows per expert on average, or one from 4096 channels (30B T=32 33.9
+/// us on the stream kernel against 36.7, T=64 37.4 against 38.7, with Zipf routing 75 against 45; 235B T=4 32.8 against 37.3, T=16 108.9 against 97.4).
 bool wide_mx_fits(const MxParams &p, bool gated, int64_t experts) {
   const int64_t lines = p.K / 256;
   constexpr int64_t kOffsetRange = int64_t{1} << 32;  // an expert's weights and the activations
   if (lines < 2 || p.n_total * (p.K / 2) >= kOffsetRange || p.routes * p.K >= kOffsetRange) return false;
   if (!gated) return p.out_width % (lines % 2 == 0 ? 256 : 512) == 0;
   return p.out_codes != nullptr && p.out_width % 128 == 0 &&
-         (p.routes > 2 * experts || (p.K >= 4096 && p.routes >= experts));
+         (p.routes > 3 * experts || (p.K >= 4096 && p.routes >= experts));
 }
 
 void launch_expert_mx(MxParams p, bool gated, const ExpertRouting &r, hipStream_t stream) {
