@@ -9,7 +9,8 @@
 // activation row. One gfx950 MFMA 16x16x128 (f8f6f4, e4m3 x e4m3) spans exactly one scale block
 // along K, so each block's product is formed exactly as the hardware accumulates it and then added
 // into the FP32 accumulator times s_w * s_x - the per-block dequantisation never touches the
-// operands. Decode shapes run the `stream` kernel; prefill shapes run the two-workgroups-per-CU
+// operands. Decode shapes run the `stream` kernel or, in the layer from about three rows per expert, the
+// `wide` one; prefill shapes run the two-workgroups-per-CU
 // kernel of grouped_dual.hpp, or, where FC1 writes its rows already quantised for FC2, the
 // one-workgroup-per-CU kernel of grouped_prefill.hpp; the quantiser's codes are bit-exact with the
 // host rule (nearest even, saturating at 448).

@@ -14,10 +14,11 @@
 // So the hardware applies both MX block scales itself and the products accumulate straight into
 // the FP32 accumulator: no per-block scaling on the VALU.
 //
-// Two product kernels, chosen by routes per expert as for the e4m3 products:
+// The product kernels, chosen by routes per expert as for the e4m3 products:
 //  * decode shapes: the stream kernel (one tile x a slice of weight rows per workgroup; weights
 //    streamed as whole 128-byte lines, non-temporal, and regrouped into the MFMA layout through
-//    each wave's own LDS buffer), walking K 256 elements (one 128-byte weight line) at a time;
+//    each wave's own LDS buffer), walking K 256 elements (one 128-byte weight line) at a time, and in
+//    the layer the wide kernel (32 activation rows by 128 weight rows per wavefront);
 //  * prefill shapes: the tiled kernel (one 128-row tile x 256 weight rows per workgroup, two
 //    workgroups per CU), both operands and both scale tables staged through LDS by DMA in two
 //    stages of 128 K.
