@@ -129,7 +129,7 @@ UNISERVE_EXTERN_C int32_t uniserve_moe_layer_no_alloc(const struct uniserve_moe_
 /// - decode sizes (at most 4096 routes over at most 512 local experts, a router of at most 1024
 ///   experts): ROUTER launches the front end - router scores and topk, plus the sort where the
 ///   layer does not skip it, plus the hidden rows' e4m3 / MXFP8 quantisation for those weights, in one
-///   kernel or (without a sort, past 8 tokens) two - and TOPK, SORT and QUANTIZE_HIDDEN launch nothing;
+///   kernel or (without a sort, past 4 tokens) two - and TOPK, SORT and QUANTIZE_HIDDEN launch nothing;
 /// - prefill sizes (at most 128 experts, hidden a multiple of 128): ROUTER launches router scores,
 ///   topk and the hidden rows' quantisation in one kernel, up to 4096 tokens in two (in a call that also
 ///   runs SORT, the sort's per-chunk counts too, so that SORT launches only its placement), TOPK launches

@@ -35,7 +35,7 @@ constexpr int64_t kTile = 128;
 constexpr int64_t kAlign = 256;
 // Tokens up to which the expert-split front end serves, and between which the one with a workgroup per
 // token does (at most one per CU).
-constexpr int64_t kSplitFrontMost = 8, kTokenFrontLeast = 32, kTokenFrontMost = 256;
+constexpr int64_t kSplitFrontMost = 4, kTokenFrontLeast = 32, kTokenFrontMost = 256;
 
 int64_t aligned(int64_t bytes) { return (bytes + kAlign - 1) / kAlign * kAlign; }
 
@@ -356,7 +356,9 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
     // then launches nothing).
     // Layers without a sort past the smallest batches: the prefill front end's split launches, except
     // where a workgroup per token has a CU to itself and rows short enough (30B T=64 11.5 us against 11.6;
-    // past one token per CU, T=301, 21.7 against 12.6; 235B T=64 17.7 against 14.9, T=16 16.1 against 14.5).
+    // past one token per CU, T=301, 21.7 against 12.6; 235B T=64 17.7 against 14.9, T=16 16.1 against 14.5) and
+    // for up to four tokens, which the expert-split front end takes one after another (T=4 11.8 us against
+    // 10.5 and a launch more; T=5 12.7 against 10.5, T=8 16.3 against 10.7, 235B MXFP4 T=8 28.7 against 16.4).
     const bool chunk_front = by_expert && call->tokens > kSplitFrontMost &&
                              (call->tokens < kTokenFrontLeast || call->tokens > kTokenFrontMost || call->hidden_size >= 4096) &&
                              prefill_front_fits(call->tokens, call->experts, call->hidden_size, call->top) &&
