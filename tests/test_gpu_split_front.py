@@ -70,3 +70,30 @@ def test_split_front_is_the_separate_operators(device, case):
         maps = ops.moe_sort(ids.contiguous(), weights.contiguous(), experts, local=(offset, offset + local), live_tokens=live_t)
         got = layer.view("expanded_to_permuted", torch.int32, (tokens * top,))
         assert torch.equal(got, maps[ops.EXPANDED_TO_PERMUTED][: tokens * top])
+
+
+@pytest.mark.parametrize("tokens", [31, 300, 900, 1100, 2000])
+def test_scores_do_not_depend_on_the_share(device, tokens):
+    """Eight, four or two workgroups share a token's experts, and all walk K from the same stage: equal
+    router rows in different shares give equal scores (so the lower expert comes first), and every score
+    is bit for bit the single-launch front end's, which serves past 4096 tokens."""
+    announce("split front, equal router rows", tokens)
+    hidden, experts, top, intermediate, most = 4096, 128, 8, 128, 4128
+    x = normal_bf16((most, hidden), 111, device=device)
+    half = normal_bf16((experts // 2, hidden), 112, 0.02, device)
+    router = torch.cat([half, half])
+    up_gate = normal_bf16((experts, 2 * intermediate, hidden), 113, 0.02, device)
+    down = normal_bf16((experts, hidden, intermediate), 114, 0.02, device)
+    scores = {}
+    for count in (tokens, most):
+        layer = ops.MoeLayer(hidden, experts, top, intermediate, count)
+        layer(x[:count], router, up_gate, down)
+        torch.cuda.synchronize()
+        scores[count] = layer.view("scores", torch.int16, (count, experts))[:tokens].clone()
+        if count == tokens:
+            ids = layer.view("ids", torch.int32, (tokens, top)).clone()
+    assert torch.equal(scores[tokens][:, : experts // 2], scores[tokens][:, experts // 2 :])
+    assert torch.equal(scores[tokens], scores[most])
+    values = scores[tokens].view(torch.bfloat16).float()
+    want = torch.sort(values, dim=1, descending=True, stable=True).indices[:, :top]  # ties: the lower expert
+    assert torch.equal(ids.long(), want)

@@ -273,7 +273,9 @@ __global__ void __launch_bounds__(kThreads) split_scores_kernel(PrefillFrontPara
   const int first = own * kOwn;
   if (own == 0 && p.chunk_counts != nullptr && static_cast<int>(threadIdx.x) < p.local_experts)
     p.chunk_counts[static_cast<int64_t>(blockIdx.x / kSplit) * p.local_experts + threadIdx.x] = 0;
-  const int rotation = static_cast<int>(blockIdx.x % static_cast<uint32_t>(stages));
+  // (The chunk's stage, one for all its shares: a token's experts must sum in one order, or equal router
+  // rows in two shares could score differently. It is also the kernel above's.)
+  const int rotation = static_cast<int>(blockIdx.x / kSplit % static_cast<uint32_t>(stages));
   auto channel_stage = [&](int k) {
     const int kk = k + rotation;
     return kk >= stages ? kk - stages : kk;
