@@ -1,5 +1,6 @@
 """Helpers of the GPU parity tests: seeded inputs, host/device moves, the comparison bars."""
 
+import ctypes
 import math
 import sys
 
@@ -7,6 +8,7 @@ import numpy as np
 import torch
 
 import oracle_lib as O
+from uniserve_moe import library
 
 
 def announce(*what):
@@ -91,3 +93,40 @@ def sort_on_host(maps, tokens, top):
         "total_padded_tokens": m[5][:1],
         "num_non_exiting_tiles": m[6][:1],
     }
+
+
+class _KernelNodeParams(ctypes.Structure):
+    """hipKernelNodeParams."""
+
+    _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                ("grid", ctypes.c_uint32 * 3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
+
+def kernels_of(call):
+    """The (mangled) names of the kernels that ``call`` launches on the current stream, in order: the
+    call is captured into a graph that never runs. It must allocate nothing."""
+    hip = library()  # (the HIP runtime's symbols resolve through the library that links it)
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    graph, count = ctypes.c_void_p(), ctypes.c_size_t()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    stream = ctypes.c_void_p(side.cuda_stream)
+    with torch.cuda.stream(side):
+        assert hip.hipStreamBeginCapture(stream, 2) == 0  # (relaxed)
+        try:
+            call()
+        finally:
+            status = hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+    assert status == 0
+    try:
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+        nodes = (ctypes.c_void_p * count.value)()
+        assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(count)) == 0
+        names = []
+        for node in nodes:
+            params = _KernelNodeParams()
+            assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
+            names.append(hip.hipKernelNameRefByPtr(ctypes.c_void_p(params.func), stream).decode())
+        return names
+    finally:
+        hip.hipGraphDestroy(graph)

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import oracle_lib as O
-from gpu_helpers import announce, assert_bf16_bar, bf16_bits, bf16_values, normal_bf16
+from gpu_helpers import announce, assert_bf16_bar, bf16_bits, bf16_values, kernels_of, normal_bf16
 from test_gpu_layer_routing import quantised
 from uniserve_moe import ops
 
@@ -82,3 +82,28 @@ def test_spread_walks_of_the_two_workgroup_kernel(device, wdtype):
     np.testing.assert_array_equal(layer.view("ids", torch.int32, (tokens, top)).cpu().numpy(), want_ids)
     assert_bf16_bar(bf16_values(out), O.bf16_decode(want_bits).astype(np.float64), wdtype,
                     max_rel=2e-2 if wdtype == "bf16" else 4e-2)
+
+
+PLAIN_WALKS = {
+    # name: weights, tokens, hidden, experts, top, intermediate, FC1 spread, FC2 spread
+    "bf16 rows of 4 KB and 2 KB": ("bf16", 768, 2048, 16, 2, 1024, True, True),
+    "bf16 rows of more than 4 KB": ("bf16", 768, 2560, 16, 2, 512, False, True),
+    "bf16, four rounds of possible FC2 items": ("bf16", 2100, 2048, 128, 8, 512, True, False),
+    "e4m3 rows of 4 KB and 1 KB": ("f8e4m3", 768, 4096, 16, 2, 1024, True, False),
+}
+
+
+@pytest.mark.parametrize("case", list(PLAIN_WALKS))
+def test_which_walks_may_be_spread(device, case):
+    wdtype, tokens, hidden, experts, top, intermediate, fc1, fc2 = PLAIN_WALKS[case]
+    announce("plain walks", case)
+    x = normal_bf16((tokens, hidden), 95, device=device)
+    router = normal_bf16((experts, hidden), 96, 0.02, device)
+    up_gate = normal_bf16((experts, 2 * intermediate, hidden), 97, 0.02, device)
+    down = normal_bf16((experts, hidden, intermediate), 98, 0.02, device)
+    *_, up_dev, down_dev, args = quantised(wdtype, up_gate, down, device)
+    layer = ops.MoeLayer(hidden, experts, top, intermediate, tokens, weight_dtype=wdtype)
+    out = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: layer(x, router, up_dev, down_dev, out=out, **args))
+    pairs = [name for name in names if "pair_kernel" in name]
+    assert ["Lb1ELb%dEE" % fc1 in pairs[0], "Lb0ELb%dEE" % fc2 in pairs[1]] == [True, True], names

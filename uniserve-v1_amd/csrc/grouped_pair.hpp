@@ -120,6 +120,14 @@ constexpr int lds_bytes() {
                                                                           : kRows * out_stride<kGated>();
 }
 
+/// Rounds of live items up to which the K walks are spread, and rounds of possible items below which the
+/// launch takes the kernel that may do so: bf16 FC2 past two rounds only loses by it (30B T=2500, 2.6
+/// rounds, 119 us against 122), e4m3 gains up to four (above).
+template <class F>
+constexpr int kMostRounds = F::kScaled ? 4 : 3;
+template <class F>
+constexpr int kSpreadBelowRounds = F::kScaled ? 6 : 4;
+
 /// e4m3 needs route-major activation scales (p.scale_rows >= the tiles' rows).
 /// kSpread: the items' K walks may start at different stages.
 template <class F, bool kGated, bool kSpread>
@@ -218,20 +226,21 @@ __global__ void __launch_bounds__(kThreads, 2) pair_kernel(PrefillParams p) {
     asm volatile("" ::"v"(sw_lanes[0]), "v"(sw_lanes[1]));
   }
 
-  // The K stage of the loop's step k. Where the live items are one to four rounds of resident
+  // The K stage of the loop's step k. Where the live items are one to kMostRounds rounds of resident
   // workgroups, each (expert, slice) starts its walk at a stage of its own and wraps around:
   // workgroups that start together would otherwise all read the same 128-byte column of their rows at
   // a time, which with row strides of whole 4 KB falls on few HBM channels. (The tiles of an expert
   // share their starts, and so their weights in L2.) A Weyl sequence over (expert, slice) spreads the
-  // starts evenly. 30B bf16 near-uniform T=450 FC1 188 -> 159 us, T=1024 194 -> 167; 235B e4m3 T=640
-  // 335 -> 297. With more rounds the items drift apart by themselves and the slices of a tile gain
-  // from reading its activation rows together (30B bf16 T=8192: 460 us, spread 474); with less than
-  // one, likewise (sixteen 235B experts, bf16 T=1024: 134, spread 142).
+  // starts evenly. 30B bf16 near-uniform T=450 FC1 194 -> 164 us, T=1024 194 -> 170, T=3000 (2.9 rounds)
+  // 217 -> 212; 235B e4m3 T=640 332 -> 304, T=1800 (3.5 rounds) 395 -> 380. With more rounds the items
+  // drift apart by themselves and the slices of a tile gain from reading its activation rows together
+  // (30B bf16 T=4096, 3.8 rounds: 264 us, spread 271); with less than one, likewise (sixteen 235B experts,
+  // bf16 T=1024: 134, spread 142).
   int start = 0;
   if constexpr (kSpread) {
     const int live_items = p.num_tiles[0] * p.slices;
     const uint32_t walk = (static_cast<uint32_t>(expert) * static_cast<uint32_t>(p.slices) + static_cast<uint32_t>(slice)) * 0x9e3779b1u;
-    if (live_items >= kResident && live_items <= 4 * kResident)
+    if (live_items >= kResident && live_items <= kMostRounds<F> * kResident)
       start = __builtin_amdgcn_readfirstlane(static_cast<int>(__umulhi(walk, static_cast<uint32_t>(stages))));
   }
   auto stage_of = [&](int k) {
@@ -554,13 +563,16 @@ inline void launch_pair(PrefillParams p, bool gated, int64_t max_tiles, hipStrea
   p.groups_per_xcd = static_cast<int32_t>(ceil_div<int64_t>(ceil_div<int64_t>(max_tiles, group), 8));
   const dim3 grid(static_cast<uint32_t>(static_cast<int64_t>(p.groups_per_xcd) * group * p.slices * 8));
   const dim3 block(static_cast<uint32_t>(pair::kThreads));
-  // Up to six rounds of resident workgroups if every tile is live: the kernel that may spread its K
-  // walks (the live tiles, which only the device knows, decide). Above, without the stage arithmetic
-  // (235B e4m3 T=4096 layer 1102 us, 1124 with it). e4m3 rows, half as long, only at whole 4 KB: the
-  // 2 KB rows of a 30B FC1 gain nothing (T=512..2048 within 1%), and keep the sums of the stand-alone
-  // products.
-  const bool spread = max_tiles * p.slices <= 6 * pair::kResident &&
-                      (!F::kScaled || p.K * F::kElementBytes % 4096 == 0);
+  // The kernel that may spread its K walks, below a few rounds of resident workgroups if every tile is
+  // live (which are, only the device knows). Above, the one without the stage arithmetic (235B e4m3
+  // T=4096 layer 1102 us, 1124 with it). By the rows' length: e4m3 only at whole 4 KB (the 2 KB rows of a
+  // 30B FC1 gain nothing, T=512..2048 within 1%, and keep the sums of the stand-alone products), bf16 only
+  // up to 4 KB (the 8 KB rows of a 235B FC1 gain 1% at 24 to 40 rows an expert, 554 -> 546 us at T=384, and
+  // their tiles' activations, read apart, cost more from there: T=1800 684 -> 716, a window of 64 experts
+  // T=2048 401 -> 435).
+  const int64_t row_bytes = p.K * F::kElementBytes;
+  const bool spread = max_tiles * p.slices < pair::kSpreadBelowRounds<F> * pair::kResident &&
+                      (F::kScaled ? row_bytes % 4096 == 0 : row_bytes <= 4096);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, p); };
   if (gated && spread) go(pair::pair_kernel<F, true, true>);
   else if (gated) go(pair::pair_kernel<F, true, false>);
