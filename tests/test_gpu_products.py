@@ -14,7 +14,8 @@ import torch
 
 import oracle_lib as O
 from gpu_helpers import (announce, assert_bf16_bar, assert_operator_bound, bf16_bits, bf16_values,
-                         normal_bf16, sort_on_host, to_bf16, zipf_bias)
+                         kernels_of, normal_bf16, sort_on_host, to_bf16, zipf_bias)
+from test_gpu_layer_routing import quantised
 from uniserve_moe import ops
 
 pytestmark = pytest.mark.gpu
@@ -43,6 +44,8 @@ CASES = {
     "235b decode one token": (1, 4096, 128, 8, 1536, "uniform"),
     "odd widths (tiled, 64-column slices)": (300, 320, 16, 4, 192, "uniform"),
     "stream, hidden not a multiple of 256 (row-sliced FC1)": (16, 320, 16, 4, 192, "uniform"),
+    "few experts of many rows (stream, two row blocks a pass)": (70, 384, 8, 2, 256, "zipf"),
+    "FC2 of an odd number of 64 columns (stream, two row blocks a pass)": (72, 192, 8, 2, 256, "uniform"),
 }
 
 
@@ -153,3 +156,54 @@ def test_router_gemm(device, tokens, experts, hidden):
     if tokens <= 64:
         np.testing.assert_allclose(got, bf16_values(to_bf16(O.router_gemm(bf16_bits(x), bf16_bits(w)), device)),
                                    rtol=2.0**-7, atol=1e-6)
+
+
+def test_two_row_blocks_where_the_wide_kernels_do_not_serve(device):
+    """Above eight rows per expert the stream kernels take two blocks of 16 rows a pass: by the sort's
+    tiles with few experts and at widths of an odd number of 64 columns, expert-major at K = 128 (bf16
+    FC2) and at widths of an odd number of 128 columns (e4m3 FC2 of 6 lines)."""
+    announce("two row blocks")
+    tokens, experts, top = 72, 8, 2
+    ids = torch.arange(tokens * top, device=device, dtype=torch.int32).reshape(tokens, top) % experts
+    maps = ops.moe_sort(ids, torch.rand((tokens, top), device=device), experts)
+    rows = ops.permuted_rows(tokens, top, experts)
+    x = normal_bf16((tokens, 384), 11, device=device)
+    up_gate = normal_bf16((experts, 512, 384), 12, 0.02, device)
+    gated = torch.zeros((rows, 256), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: ops.gather_gemm(x, up_gate, top, maps, rows, out=gated))
+    assert "stream_kernelILb1ELi2ELb0EE" in names[-1], names
+    down = normal_bf16((experts, 192, 256), 13, 0.02, device)
+    products = torch.zeros((rows, 192), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: ops.route_gemm(gated, down, maps, out=products))
+    assert "stream_kernelILb0ELi2ELb0EE" in names[-1], names
+
+
+BY_EXPERT_TWO_BLOCKS = {
+    # weights: tokens, hidden, experts, top, intermediate, FC2's kernel
+    "bf16": (140, 640, 128, 8, 128, "stream_kernelILb0ELi2ELb1EE"),
+    "f8e4m3": (140, 640, 128, 8, 768, "stream_fp8_kernelILb0ELb0ELi2ELb1ELi1ELi4ELb0EE"),
+}
+
+
+@pytest.mark.parametrize("wdtype", list(BY_EXPERT_TWO_BLOCKS))
+def test_expert_major_two_row_blocks(device, wdtype):
+    tokens, hidden, experts, top, intermediate, kernel = BY_EXPERT_TWO_BLOCKS[wdtype]
+    announce("expert-major two row blocks", wdtype)
+    x = normal_bf16((tokens, hidden), 14, device=device)
+    router = normal_bf16((experts, hidden), 15, 0.02, device)
+    up_gate = normal_bf16((experts, 2 * intermediate, hidden), 16, 0.02, device)
+    down = normal_bf16((experts, hidden, intermediate), 17, 0.02, device)
+    bias = zipf_bias(experts)
+    bias_dev = torch.from_numpy(bias).to(device)
+    w1, w2, s1, s2, up_dev, down_dev, args = quantised(wdtype, up_gate, down, device)
+    layer = ops.MoeLayer(hidden, experts, top, intermediate, tokens, weight_dtype=wdtype)
+    out = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: layer(x, router, up_dev, down_dev, out=out, router_bias=bias_dev, **args))
+    assert any(kernel in name for name in names), names
+    layer(x, router, up_dev, down_dev, out=out, router_bias=bias_dev, **args)
+    torch.cuda.synchronize()
+    want_bits, want_ids, _, _ = O.moe_layer(bf16_bits(x), bf16_bits(router), w1, w2, top, up_gate_scales=s1,
+                                            down_scales=s2, router_bias=bias)
+    np.testing.assert_array_equal(layer.view("ids", torch.int32, (tokens, top)).cpu().numpy(), want_ids)
+    assert_bf16_bar(bf16_values(out), O.bf16_decode(want_bits).astype(np.float64), wdtype,
+                    max_rel=2e-2 if wdtype == "bf16" else 4e-2)

@@ -18,8 +18,9 @@
 //    every touched expert's matrix is read from HBM and little else matters. A workgroup owns 128
 //    weight rows and 32 activation rows, its wavefronts a quarter of K each.
 //
-//  * `stream` (FC2 of the smallest batches, and K below 256): a 128-row slice of the expert's weight
-//    rows per workgroup, each wavefront streaming its own 32 rows over all of K. The weight lines are
+//  * `stream` (FC2 of the smallest batches, FC2 widths of an odd number of 64 columns, few experts, and K
+//    below 256): a 128-row slice of the expert's weight rows per workgroup, each wavefront streaming its
+//    own 32 rows over all of K. The weight lines are
 //    regrouped into the MFMA operand layout through LDS, the activation rows come from L2. The weight
 //    rows are MFMA operand A and the activation rows operand B (16x16x32 bf16), so each lane ends
 //    holding four consecutive output columns of one row - an 8-byte store - and the SiLU pair (up
@@ -87,6 +88,13 @@ __device__ __forceinline__ void store_bf16x4(uint16_t *pointer, floatx4 v) {
 
 // ---- stream kernel (decode) ----------------------------------------------------------------------------
 
+/// Average routes per expert at or below which the stream kernel takes its rows in passes of one
+/// 16-row MFMA block instead of two (64-token decode: FC2 63.7 against 66.2 us with two); an expert with
+/// more rows re-streams its weights per pass, which at such averages is rare. Above, two (FC2 of 1984
+/// columns by tiles, 128 experts, T=300: 124 us with one, 82 with two; FC1 of 8 experts, 30B widths, T=90:
+/// 35.5 against 24.1; expert-major FC2 of 128 channels T=300: 30 against 23).
+constexpr int64_t kOnePassRowsPerExpert = 8;
+
 //
 // Grid: (max tiles, weight-row slices). FC1 slices are 64 gated columns (64 up + 64 gate rows),
 // FC2 slices 128 output columns; wavefront w takes 16 + 16 of them. Needs K % 128 == 0.
@@ -102,14 +110,14 @@ __device__ __forceinline__ void store_bf16x4(uint16_t *pointer, floatx4 v) {
 // K mapping (the same for weights and activations): step s in 0..3 of a stage, lane group
 // g = l / 16 takes the stage's 16-byte chunk 4 s + g, i.e. line s / 2, chunk 4 (s % 2) + g.
 
+/// kPassTiles: rows one pass covers, in MFMA blocks of 16.
 /// kByExpert: workgroup x serves local expert x (grid: local experts x slices) and finds its rows
 /// itself - the routes whose id is the expert's, in route order, live ones only (each wavefront
 /// ballots a quarter of the routes into a list in LDS) - while its first weight stage is in
 /// flight; FC1 reads token route / top and FC2 row `route`, and both write row `route` (the
 /// expanded layout). Otherwise the sort's tile tables give the tile's expert and rows.
-template <bool kGated, bool kByExpert>
+template <bool kGated, int kPassTiles, bool kByExpert>
 __global__ void __launch_bounds__(kThreads) stream_kernel(GroupedParams p) {
-  constexpr int kPassTiles = 1;  // 16-row MFMA blocks per pass
   const int wave = static_cast<int>(threadIdx.x) / kWave;
   const int lane = lane_id();
   const int r16 = lane & 15;
@@ -643,7 +651,10 @@ bool wide_fits(const GroupedParams &p, int64_t act_rows) {
 }
 
 template <bool kGated>
-void launch_grouped(const GroupedParams &p, int64_t max_tiles, int64_t act_rows, bool stream_path, bool few_rows, hipStream_t s) {
+void launch_grouped(const GroupedParams &p, int64_t max_tiles, int64_t act_rows, int64_t routes, int64_t experts, hipStream_t s) {
+  const bool stream_path = routes < kStreamRowsPerExpert * experts && p.K % 128 == 0;
+  const bool few_rows = !kGated && routes <= kWideFc2RowsPerExpert * experts;
+
   if (!stream_path && (pair_fits<pair::Bf16>(kGated, p.K, p.out_width, 0) || prefill_fits<prefill::Bf16, kGated>(p.K, p.out_width))) {
     PrefillParams q{};
     q.act = reinterpret_cast<const uint8_t *>(p.act);
@@ -669,7 +680,9 @@ void launch_grouped(const GroupedParams &p, int64_t max_tiles, int64_t act_rows,
   if (stream_path && max_tiles * slices >= kWideWorkgroups && (kGated || (!few_rows && p.out_width % 128 == 0)) &&
       wide_fits(p, act_rows))
     hipLaunchKernelGGL((wide_kernel<kGated, false>), grid, dim3(kThreads), 0, s, p);
-  else if (stream_path) hipLaunchKernelGGL((stream_kernel<kGated, false>), grid, dim3(kThreads), 0, s, p);
+  else if (stream_path && routes <= kOnePassRowsPerExpert * experts)
+    hipLaunchKernelGGL((stream_kernel<kGated, 1, false>), grid, dim3(kThreads), 0, s, p);
+  else if (stream_path) hipLaunchKernelGGL((stream_kernel<kGated, 2, false>), grid, dim3(kThreads), 0, s, p);
   else hipLaunchKernelGGL(tiled_kernel<kGated>, grid, dim3(kThreads), 0, s, p);
 }
 
@@ -717,8 +730,11 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
     else hipLaunchKernelGGL((wide_kernel<false, true>), wide_grid, dim3(kThreads), 0, stream, p);
     return;
   }
-  if (gated) hipLaunchKernelGGL((stream_kernel<true, true>), grid, dim3(kThreads), 0, stream, p);
-  else hipLaunchKernelGGL((stream_kernel<false, true>), grid, dim3(kThreads), 0, stream, p);
+  const bool one_pass = e.routes <= kOnePassRowsPerExpert * e.local_experts;
+  if (gated && one_pass) hipLaunchKernelGGL((stream_kernel<true, 1, true>), grid, dim3(kThreads), 0, stream, p);
+  else if (gated) hipLaunchKernelGGL((stream_kernel<true, 2, true>), grid, dim3(kThreads), 0, stream, p);
+  else if (one_pass) hipLaunchKernelGGL((stream_kernel<false, 1, true>), grid, dim3(kThreads), 0, stream, p);
+  else hipLaunchKernelGGL((stream_kernel<false, 2, true>), grid, dim3(kThreads), 0, stream, p);
 }
 
 int32_t gather_gemm_bf16(const uniserve_gather_call *call, int32_t activation, void *stream) {
@@ -766,9 +782,7 @@ int32_t gather_gemm_bf16(const uniserve_gather_call *call, int32_t activation, v
     p.out_width = call->width / 2;
     p.top = call->top;
     p.activation = activation;
-    const bool stream_path = call->tokens * call->top < kStreamRowsPerExpert * call->experts &&
-                             call->hidden_size % 128 == 0;
-    launch_grouped<true>(p, max_tiles, call->tokens, stream_path, false, static_cast<hipStream_t>(stream));
+    launch_grouped<true>(p, max_tiles, call->tokens, call->tokens * call->top, call->experts, static_cast<hipStream_t>(stream));
     return launched(call, "gather_gemm");
   });
 }
@@ -820,10 +834,7 @@ extern "C" int32_t uniserve_route_gemm(const uniserve_route_call *call, void *st
     // The call states no token count: the permuted rows bound the routes, and their expected
     // share per expert is (rows - the padding of one partial tile per expert) / experts.
     const int64_t routes_bound = call->permuted_rows - (kTileRows - 1) * call->experts;
-    const bool stream_path = routes_bound < kStreamRowsPerExpert * call->experts &&
-                             call->intermediate % 128 == 0;
-    launch_grouped<false>(p, max_tiles, kTileRows, stream_path, routes_bound <= kWideFc2RowsPerExpert * call->experts,
-                          static_cast<hipStream_t>(stream));
+    launch_grouped<false>(p, max_tiles, kTileRows, routes_bound, call->experts, static_cast<hipStream_t>(stream));
     return launched(call, "route_gemm");
   });
 }
