@@ -107,3 +107,51 @@ def test_which_walks_may_be_spread(device, case):
     names = kernels_of(lambda: layer(x, router, up_dev, down_dev, out=out, **args))
     pairs = [name for name in names if "pair_kernel" in name]
     assert ["Lb1ELb%dEE" % fc1 in pairs[0], "Lb0ELb%dEE" % fc2 in pairs[1]] == [True, True], names
+
+
+_FC1 = {"f8e4m3": "wide_fp8_kernelILb1ELi2ELi2ELb1EE", "f4e2m1": "wide_mx_kernelILb1ELi2ELi2ELb1EE"}
+WIDE = {
+    # name: weights, tokens, hidden, experts, top, intermediate, window, live, FC2's kernel. (At most 48
+    # runs past the first passes are shared out to columns of their own: eight experts of 300 rows have 72
+    # and take them 64 rows at a time, of 288 rows 64.)
+    "e4m3, window, FC2 of 4 lines": ("f8e4m3", 300, 1024, 128, 8, 512, (0, 16), None, "wide_fp8_kernelILb0ELi4ELi1ELb0EE"),
+    "e4m3, window, FC2 of 6 lines": ("f8e4m3", 288, 2048, 128, 8, 768, (0, 16), None, "wide_fp8_kernelILb0ELi2ELi2ELb0EE"),
+    "e4m3, window, some rows not live": ("f8e4m3", 200, 1024, 128, 8, 512, (4, 20), 150, "wide_fp8_kernelILb0ELi4ELi1ELb0EE"),
+    "mx, window, FC2 of 2 lines": ("f4e2m1", 300, 1024, 128, 8, 512, (0, 16), None, "wide_mx_kernelILb0ELi2ELi2ELb0EE"),
+    "mx, window, FC2 of 3 lines": ("f4e2m1", 288, 2048, 128, 8, 768, (0, 16), None, "wide_mx_kernelILb0ELi1ELi4ELb0EE"),
+    "mx, window, some rows not live": ("f4e2m1", 200, 1024, 128, 8, 768, (4, 20), 150, "wide_mx_kernelILb0ELi1ELi4ELb0EE"),
+    "bf16, window": ("bf16", 300, 512, 128, 8, 256, (0, 16), None, "wide_kernelILb0ELb1ELi2EE"),
+}
+
+
+@pytest.mark.parametrize("case", list(WIDE))
+def test_wide_kernels_share_out_a_windows_rows(device, case):
+    """A window that holds the much-named experts takes the wide kernels, whose further columns share out
+    the rows past an expert's first pass."""
+    wdtype, tokens, hidden, experts, top, intermediate, window, live, fc2 = WIDE[case]
+    announce("wide kernels, window", case)
+    x = normal_bf16((tokens, hidden), 101, device=device)
+    router = normal_bf16((experts, hidden), 102, 0.02, device)
+    up_gate = normal_bf16((window[1], 2 * intermediate, hidden), 103, 0.02, device)
+    down = normal_bf16((window[1], hidden, intermediate), 104, 0.02, device)
+    bias = np.where(np.arange(experts) < top, 40.0, 0.0).astype(np.float32)
+    bias_dev = torch.from_numpy(bias).to(device)
+    live_t = None if live is None else torch.tensor([live], dtype=torch.int32, device=device)
+    w1, w2, s1, s2, up_dev, down_dev, args = quantised(wdtype, up_gate, down, device)
+    layer = ops.MoeLayer(hidden, experts, top, intermediate, tokens, weight_dtype=wdtype)
+    out = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=device)
+
+    def call():
+        layer(x, router, up_dev, down_dev, out=out, router_bias=bias_dev, live_tokens=live_t, window=window, **args)
+
+    names = kernels_of(call)
+    fc1 = _FC1.get(wdtype, "wide_kernelILb1ELb1ELi2EE")
+    assert any(fc1 in name for name in names) and any(fc2 in name for name in names), names
+    call()
+    torch.cuda.synchronize()
+    want_bits, want_ids, _, _ = O.moe_layer(bf16_bits(x), bf16_bits(router), w1, w2, top, up_gate_scales=s1,
+                                            down_scales=s2, router_bias=bias, live=live, window=window)
+    served = tokens if live is None else live
+    np.testing.assert_array_equal(layer.view("ids", torch.int32, (tokens, top)).cpu().numpy()[:served], want_ids[:served])
+    assert_bf16_bar(bf16_values(out)[:served], O.bf16_decode(want_bits).astype(np.float64)[:served], case,
+                    max_rel=2e-2 if wdtype == "bf16" else 4e-2)

@@ -103,6 +103,7 @@ __device__ __forceinline__ void store_bf16x4(uint16_t *pointer, floatx4 v) {
 constexpr int64_t kOnePassRowsPerExpert = 8;
 
 constexpr int64_t kSplitBelow = 512;  // stream workgroups under which K is split over the waves
+constexpr int64_t kWideExperts = 16;  // expert-major: experts from which the wide kernel may take such products
 
 /// Decode-shaped: as the bf16 stream kernel, one 128-deep scale block per chunk. kSplit: the four
 /// wavefronts share one row set and split K (scale block kb goes to wave kb % 4), their partial sums
@@ -834,11 +835,6 @@ bool fp8_stream_path(int64_t routes, int64_t experts) { return routes < kStreamR
 /// 15.9 us by events with two (four: 23.2).
 constexpr int kSplitFc2Run = 2;
 
-bool expert_stream_fp8_fc1_quantizes(int64_t routes, int64_t local_experts, int64_t out_width) {
-  const int64_t served = routes < local_experts ? routes : local_experts;
-  return served * (out_width / 64) >= kSplitBelow && out_width % 128 == 0;
-}
-
 /// Whether the wide kernel takes the unsplit expert-major product (p.experts, the router's): above two
 /// (FC1: three) rows per expert on average, and FC1 from 4096 channels at any (235B T=4 68 -> 62 us, T=16
 /// 186 -> 171); below, the stream kernel's workgroups need no exchange of partial sums (30B T=32 FC1 59.0 us
@@ -849,20 +845,35 @@ bool wide_fp8_fits(const GroupedFp8Params &p, bool gated) {
   constexpr int64_t kOffsetRange = int64_t{1} << 32;
   const int64_t lines = p.K / 128;
   const bool rows = p.routes > (gated ? 3 : 2) * p.experts || (gated && lines >= 32);
-  return rows && (gated ? p.out_codes != nullptr : lines % 4 == 0 || p.out_width % 256 == 0) && lines >= 2 &&
+  return rows && (gated ? p.out_width % 128 == 0 : lines % 4 == 0 || p.out_width % 256 == 0) && lines >= 2 &&
          lines <= 128 && p.n_total * p.K < kOffsetRange && p.routes * p.K < kOffsetRange;
 }
 
-void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, int64_t local_experts, hipStream_t stream) {
+/// Whether the expert-major product splits K over the wavefronts (16 or 32 output columns a workgroup):
+/// where larger slices would be fewer than two workgroups per CU - unless an expert may have more than two
+/// wide passes of rows, which a split workgroup takes one after the other and the wide kernel shares out.
+/// Layer, sixteen of 128 experts from the first, Zipf, split -> wide: 30B T=100 94 -> 57 us, T=383 252 ->
+/// 119, 235B 198 -> 131 and 688 -> 320; near-uniform 30B T=200 50 -> 50, 235B 96 -> 89. Up to 64 tokens the
+/// wide kernel shares nothing out (30B T=64 Zipf 66 -> 76), and eight experts' columns are too few for it (T=200
+/// near-uniform 40 -> 46, 235B 66 -> 78).
+bool split_fp8(const GroupedFp8Params &p, bool gated) {
+  // Workgroups with routes: at most one per route.
+  const int64_t served = p.routes < p.local_experts ? p.routes : p.local_experts;
+  if (served * (p.out_width / (gated ? 64 : 128)) >= kSplitBelow) return false;
+  const bool shared_out = p.local_experts >= kWideExperts && p.routes > 2 * kWideRows * p.top;
+  return !(shared_out && wide_fp8_fits(p, gated));
+}
+
+bool expert_stream_fp8_fc1_quantizes(const GroupedFp8Params &p) { return !split_fp8(p, true) && p.out_width % 128 == 0; }
+
+void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, hipStream_t stream) {
   GroupedFp8Params p = params;
-  p.local_experts = local_experts;
+  const int64_t local_experts = p.local_experts;
   p.compact = p.routes < local_experts ? 1 : 0;
   const int64_t columns = p.compact ? p.routes : local_experts;  // workgroup columns
   const bool one_pass = p.routes <= kOnePassRowsPerExpert * local_experts;
   const int64_t slices = gated ? p.out_width / 64 : p.out_width / 128;
-  // Workgroups with routes: at most one per route.
-  const int64_t served = p.routes < local_experts ? p.routes : local_experts;
-  if (served * slices < kSplitBelow) {
+  if (split_fp8(p, gated)) {
     const dim3 grid(static_cast<uint32_t>(columns), static_cast<uint32_t>(gated ? p.out_width / 16 : p.out_width / 32));
     const dim3 run_grid(static_cast<uint32_t>(columns), static_cast<uint32_t>(p.out_width / 32 / kSplitFc2Run));
     const bool runs = !gated && (p.out_width / 32) % kSplitFc2Run == 0;

@@ -102,6 +102,7 @@ constexpr int kTileRows = 128;
 constexpr int kThreads = 256;
 constexpr int kPassTiles = 1;           // 16-token MFMA blocks per pass (one keeps three waves per SIMD)
 constexpr int64_t kSplitBelow = 512;    // workgroups under which K is split over the waves
+constexpr int64_t kWideExperts = 16;    // expert-major: experts from which the wide kernel may take such products
 
 struct MxParams {
   const uint8_t *act;            ///< FC1: [tokens, K] e4m3; FC2: [permuted_rows, K]
@@ -1182,8 +1183,23 @@ bool wide_mx_fits(const MxParams &p, bool gated, int64_t experts) {
   constexpr int64_t kOffsetRange = int64_t{1} << 32;  // an expert's weights and the activations
   if (lines < 2 || p.n_total * (p.K / 2) >= kOffsetRange || p.routes * p.K >= kOffsetRange) return false;
   if (!gated) return p.out_width % (lines % 2 == 0 ? 256 : 512) == 0;
-  return p.out_codes != nullptr && p.out_width % 128 == 0 &&
-         (p.routes > 3 * experts || (p.K >= 4096 && p.routes >= experts));
+  return p.out_width % 128 == 0 && (p.routes > 3 * experts || (p.K >= 4096 && p.routes >= experts));
+}
+
+/// Whether the expert-major product splits K over the wavefronts (16 or 32 output columns a workgroup):
+/// where larger slices would be fewer than two workgroups per CU - unless an expert may have more than two
+/// wide passes of rows, which a split workgroup takes 16 at a time and the wide kernel shares out. Layer,
+/// sixteen of 128 experts from the first, Zipf, split -> wide: 30B T=200 137 -> 62 us, T=383 230 -> 92, 235B
+/// T=100 177 -> 91, T=383 607 -> 215; near-uniform 30B T=200 42 -> 43, T=383 54 -> 50, 235B T=100 63 -> 57. Fewer
+/// than 32 experts with rows of less than 4096 channels only above eight per expert (30B T=100 near-uniform
+/// 37.5 -> 40; 32 experts 47 -> 41), and not eight experts, whose columns are too few (T=200 38 -> 41).
+bool split_mx(const MxParams &p, bool gated, int64_t experts) {
+  // Workgroups with routes: at most one per route.
+  const int64_t served = p.routes < p.local_experts ? p.routes : p.local_experts;
+  if (served * (p.out_width / (gated ? 64 : 128)) >= kSplitBelow) return false;
+  const bool shared_out = p.local_experts >= kWideExperts && p.routes > 2 * kWideRows * p.top &&
+                          (p.K >= 4096 || p.local_experts >= 2 * kWideExperts || p.routes > 8 * experts);
+  return !(shared_out && wide_mx_fits(p, gated, experts));
 }
 
 void launch_expert_mx(MxParams p, bool gated, const ExpertRouting &r, hipStream_t stream) {
@@ -1195,8 +1211,7 @@ void launch_expert_mx(MxParams p, bool gated, const ExpertRouting &r, hipStream_
   p.compact = r.routes < r.local_experts ? 1 : 0;
   const int64_t columns = p.compact ? r.routes : r.local_experts;
   const int64_t slices = gated ? p.out_width / 64 : p.out_width / 128;
-  const int64_t served = r.routes < r.local_experts ? r.routes : r.local_experts;
-  if (served * slices < kSplitBelow) {
+  if (split_mx(p, gated, r.experts)) {
     const dim3 grid(static_cast<uint32_t>(columns), static_cast<uint32_t>(gated ? p.out_width / 16 : p.out_width / 32));
     if (gated) {
       hipLaunchKernelGGL((stream_mx_kernel<true, true, true>), grid, dim3(kThreads), 0, stream, p);
@@ -1236,9 +1251,15 @@ void launch_expert_mx(MxParams p, bool gated, const ExpertRouting &r, hipStream_
 
 }  // namespace
 
-bool mx_fc1_quantizes_by_expert(const ExpertRouting &r, int64_t width) {
-  const int64_t served = r.routes < r.local_experts ? r.routes : r.local_experts;
-  return served * (width / 2 / 64) >= kSplitBelow;
+bool mx_fc1_quantizes_by_expert(const ExpertRouting &r, int64_t width, int64_t hidden_size) {
+  MxParams p{};
+  p.routes = r.routes;
+  p.top = r.top;
+  p.local_experts = r.local_experts;
+  p.K = hidden_size;
+  p.n_total = width;
+  p.out_width = width / 2;
+  return !split_mx(p, true, r.experts);
 }
 
 void gather_gemm_mx_by_expert(const uniserve_gather_mx_call *call, const ExpertRouting &r, int32_t activation,

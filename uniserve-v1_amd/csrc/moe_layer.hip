@@ -240,7 +240,7 @@ int32_t run_mx_products(const uniserve_moe_layer_call *call, const uniserve_moe_
   fc1.weight_scale_layout = call->weight_scale_layout;
   // Decode sizes on the unsplit kernel: FC1 also writes FC2's MXFP8 operand (QUANTIZE_GATED then
   // launches nothing).
-  const bool fc1_quantizes = by_expert != nullptr && mx_fc1_quantizes_by_expert(*by_expert, 2 * call->intermediate);
+  const bool fc1_quantizes = by_expert != nullptr && mx_fc1_quantizes_by_expert(*by_expert, 2 * call->intermediate, call->hidden_size);
   if (!want(UNISERVE_MOE_LAYER_GATHER)) {
   } else if (by_expert != nullptr) {
     gather_gemm_mx_by_expert(&fc1, *by_expert, static_cast<int32_t>(call->activation), stream,
@@ -670,11 +670,15 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
         e.experts = call->experts;
         e.top = call->top;
         e.activation = activation;
-        // Where the unsplit kernel serves FC1 it also writes FC2's operand (QUANTIZE_GATED then
+        e.local_experts = local_experts;
+        // Where the unsplit kernels serve FC1 they also write FC2's operand (QUANTIZE_GATED then
         // launches nothing).
-        const bool fc1_quantizes = expert_stream_fp8_fc1_quantizes(routes, local_experts, call->intermediate);
+        GroupedFp8Params fc1 = e;
+        fc1.K = call->hidden_size;
+        fc1.n_total = 2 * call->intermediate;
+        fc1.out_width = call->intermediate;
+        const bool fc1_quantizes = expert_stream_fp8_fc1_quantizes(fc1);
         if (want(UNISERVE_MOE_LAYER_GATHER)) {
-          GroupedFp8Params fc1 = e;
           if (fc1_quantizes) {
             fc1.out_codes = static_cast<uint8_t *>(at(v.gated_q));
             fc1.out_code_scales = static_cast<float *>(at(v.gated_s));
@@ -684,10 +688,7 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
           fc1.weights = static_cast<const uint8_t *>(call->up_gate);
           fc1.weight_scales = call->up_gate_scales;
           fc1.out = static_cast<uint16_t *>(at(v.gated));
-          fc1.K = call->hidden_size;
-          fc1.n_total = 2 * call->intermediate;
-          fc1.out_width = call->intermediate;
-          launch_expert_stream_fp8(fc1, true, local_experts, s);
+          launch_expert_stream_fp8(fc1, true, s);
           if (int32_t status = launched(call, "gather_gemm_fp8")) return status;
         }
         if (want(UNISERVE_MOE_LAYER_QUANTIZE_GATED) && !fc1_quantizes) {
@@ -705,7 +706,7 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
           fc2.K = call->intermediate;
           fc2.n_total = call->hidden_size;
           fc2.out_width = call->hidden_size;
-          launch_expert_stream_fp8(fc2, false, local_experts, s);
+          launch_expert_stream_fp8(fc2, false, s);
           if (int32_t status = launched(call, "route_gemm_fp8")) return status;
         }
       } else {
