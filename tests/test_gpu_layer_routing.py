@@ -229,15 +229,15 @@ def test_tiny_config_against_the_fp32_oracle(device):
 
 
 @pytest.mark.parametrize("garbage", [1000, 3])
-@pytest.mark.parametrize("tokens", [64, 1])
+@pytest.mark.parametrize("tokens", [64, 1, 8, 300])
 def test_uncleared_front_counters_fail_loudly_then_clear(device, garbage, tokens):
     """A decode-size call whose workspace counters were not zero before it (a reused buffer): the
     output is NaN, not a quietly wrong result, the counters are cleared, and the next call is
     bit-for-bit the clean one. Garbage past the takers means no workgroup routes; garbage below it
     means a workgroup routes early (on the previous call's scores, here the same ones). The
     workspace still holds the first call's maps, so no kernel reads outside its arrays either way.
-    At 64 tokens the front end counts nothing (the words are only checked); at one token the
-    expert-split front end counts its workgroups on word 1."""
+    At 64 tokens the front end counts nothing (the words are only checked), nor do the two launches
+    of 8 and 300 tokens; at one token the expert-split front end counts its workgroups on word 1."""
     hidden, experts, top, intermediate = 2048, 128, 8, 768
     x = normal_bf16((tokens, hidden), 71, device=device)
     router = normal_bf16((experts, hidden), 72, 0.02, device)

@@ -789,10 +789,11 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
     combine.output_dtype = UNISERVE_DTYPE_BF16;
     combine.layout = by_expert ? UNISERVE_UNPERMUTE_LAYOUT_EXPANDED : UNISERVE_UNPERMUTE_LAYOUT_PERMUTED;
     // After the fused front end the combine also checks that the front end's counters came back to
-    // zero (they do unless they were not zero before it: a workspace whose head was not cleared).
-    uint32_t *ticket = front && !chunk_front ? static_cast<uint32_t *>(at(v.ticket)) : nullptr;
+    // zero (they do unless they were not zero before it: a workspace whose head was not cleared), also
+    // where the front end counts nothing: the next call's may.
+    uint32_t *ticket = front ? static_cast<uint32_t *>(at(v.ticket)) : nullptr;
     if (want(UNISERVE_MOE_LAYER_UNPERMUTE) &&
-        moe_unpermute_checked(&combine, ticket, ticket != nullptr ? front_ticket_words(call->tokens) : 0, stream) != 0)
+        moe_unpermute_checked(&combine, ticket, front ? front_ticket_words(call->tokens) : 0, stream) != 0)
       return forward_error(call, "moe_unpermute", combine);
     return 0;
   });
