@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle_lib as O
-from gpu_helpers import announce, bf16_bits, bf16_values, normal_bf16
+from gpu_helpers import announce, bf16_bits, bf16_values, kernels_of, normal_bf16
 from test_gpu_layer_routing import quantised
 from uniserve_moe import ops
 
@@ -23,7 +23,8 @@ CASES = {
     "700 tokens, eight shares of 60 experts + live": (700, 512, 60, 8, "bf16", None, 699),
     "1025 tokens, four shares": (1025, 512, 128, 8, "f8e4m3", None, None),
     "1536 tokens, four shares of 33 experts": (1536, 256, 33, 6, "f8e4m3", None, 1500),
-    "1537 tokens, two shares": (1537, 512, 128, 8, "f4e2m1", (8, 112), None),
+    "2048 tokens, four shares": (2048, 512, 128, 8, "f4e2m1", (8, 112), None),
+    "2049 tokens, two shares": (2049, 512, 128, 8, "f4e2m1", (8, 112), None),
 }
 
 
@@ -72,7 +73,7 @@ def test_split_front_is_the_separate_operators(device, case):
         assert torch.equal(got, maps[ops.EXPANDED_TO_PERMUTED][: tokens * top])
 
 
-@pytest.mark.parametrize("tokens", [31, 300, 900, 1100, 2000])
+@pytest.mark.parametrize("tokens", [31, 300, 900, 1100, 2000, 2100])
 def test_scores_do_not_depend_on_the_share(device, tokens):
     """Eight, four or two workgroups share a token's experts, and all walk K from the same stage: equal
     router rows in different shares give equal scores (so the lower expert comes first), and every score
@@ -97,3 +98,23 @@ def test_scores_do_not_depend_on_the_share(device, tokens):
     values = scores[tokens].view(torch.bfloat16).float()
     want = torch.sort(values, dim=1, descending=True, stable=True).indices[:, :top]  # ties: the lower expert
     assert torch.equal(ids.long(), want)
+
+
+@pytest.mark.parametrize("wdtype", ["bf16", "f8e4m3", "f4e2m1"])
+@pytest.mark.parametrize("tokens, shares", [(1024, 8), (1025, 4), (2048, 4), (2049, 2), (4096, 2), (4097, 1)])
+def test_shares_fill_the_chip_once(device, tokens, shares, wdtype):
+    """Eight, four or two workgroups per 32 tokens, at most 256 in all, whatever the weights; one where
+    the tokens alone make more than 128."""
+    announce("split front, shares", tokens, wdtype)
+    hidden, experts, top, intermediate = 512, 32, 8, 256
+    x = normal_bf16((tokens, hidden), 121, device=device)
+    router = normal_bf16((experts, hidden), 122, 0.02, device)
+    up_gate = normal_bf16((experts, 2 * intermediate, hidden), 123, 0.02, device)
+    down = normal_bf16((experts, hidden, intermediate), 124, 0.02, device)
+    *_, up_dev, down_dev, args = quantised(wdtype, up_gate, down, device)
+    layer = ops.MoeLayer(hidden, experts, top, intermediate, tokens, weight_dtype=wdtype)
+    out = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: layer(x, router, up_dev, down_dev, out=out, **args))
+    quant = {"bf16": 0, "f8e4m3": 1, "f4e2m1": 2}[wdtype]
+    want = f"split_scores_kernelILi{quant}ELi{shares}EE" if shares > 1 else f"prefill_front_kernelILi{quant}EE"
+    assert want in names[0], names

@@ -410,12 +410,14 @@ bool prefill_front_fits(int64_t tokens, int64_t experts, int64_t hidden, int64_t
          ceil_div<int64_t>(tokens, kTokens) <= 0x7fffffffLL;
 }
 
-/// Workgroups that share 32 tokens: as many as fill the 256 CUs once (two from 49 chunks, where the
-/// shared hidden rows cost more than four would gain: 30B bf16 T=2048 10.5 us against 12.1), one where the
-/// chunks fill them by themselves (T=8192: 30 us either way, and a launch more).
+/// Workgroups that share 32 tokens: as many as fill the 256 CUs once (four against two at T=2048, layer of
+/// sixteen held experts: 30B e4m3 81 us against 84, MXFP4 70 against 73, bf16 94.5 either way, 235B e4m3 168
+/// against 173, MXFP4 136 against 141, bf16 243 against 245; at T=2560 MXFP4 77 against 75, 235B 149 against
+/// 146, bf16 100 against 97), one where the chunks fill them by themselves (T=8192: 30 us either way, and a
+/// launch more).
 int prefill_front_split(int64_t tokens) {
   const int64_t chunks = ceil_div<int64_t>(tokens, kTokens);
-  return chunks <= 32 ? 8 : chunks <= 48 ? 4 : chunks <= 128 ? 2 : 1;
+  return chunks <= 32 ? 8 : chunks <= 64 ? 4 : chunks <= 128 ? 2 : 1;
 }
 
 void launch_prefill_front(const PrefillFrontParams &p, hipStream_t stream) {
