@@ -15,7 +15,7 @@ import pytest
 import torch
 
 import oracle_lib as O
-from gpu_helpers import (announce, assert_bf16_bar, bf16_bits, bf16_values, normal_bf16, sort_on_host,
+from gpu_helpers import (announce, assert_bf16_bar, bf16_bits, bf16_values, kernels_of, normal_bf16, sort_on_host,
                          zipf_bias)
 from uniserve_moe import ops
 
@@ -49,17 +49,42 @@ ROUTED = {
     "bf16 8 tokens, map + load + window + live": (8, 2048, 128, 8, 768, "bf16", (16, 96), 6),
     "fp8 8 tokens, map + load + window": (8, 2048, 128, 8, 768, "f8e4m3", (16, 96), None),
     "mx 8 tokens, map + load + window": (8, 2048, 128, 8, 768, "f4e2m1", (16, 96), None),
-    # the expert-split front end (at most 8 tokens) off its usual shape: an expert count that is
-    # no multiple of its four experts per workgroup, one or three 512-channel chunks of a narrow
-    # row, five of a wide one, top 10
+    # the two-launch front end of 5 to 31 tokens, and the expert-split one (at most 4 tokens), off their
+    # usual shape: an expert count that is no multiple of the experts per workgroup, one or three
+    # 512-channel chunks of a narrow row, five of a wide one, top 10
     "fp8 5 tokens, 60 experts, 512 channels": (5, 512, 60, 4, 256, "f8e4m3", None, None),
     "mx 3 tokens, 1536 channels, window + live": (3, 1536, 128, 8, 512, "f4e2m1", (8, 64), 2),
     "bf16 7 tokens, 100 experts, top 10, 2560 channels": (7, 2560, 100, 10, 384, "bf16", None, None),
-    # a window of 16 experts: 24 or more routes per local expert, so the decode front end (which
-    # still quantises the hidden rows) hands over to the sort and the tiled products
+    "fp8 4 tokens, 60 experts, 512 channels": (4, 512, 60, 4, 256, "f8e4m3", None, None),
+    "bf16 4 tokens, 100 experts, top 10, 2560 channels": (4, 2560, 100, 10, 384, "bf16", None, None),
+    # more experts than either takes: the tile-split front end with tickets, without a sort
+    "mx 7 tokens, 160 experts": (7, 512, 160, 8, 256, "f4e2m1", None, None),
+    # a window of 16 experts: its products go without a sort in few workgroups
     "fp8 decode, narrow window": (64, 2048, 128, 8, 768, "f8e4m3", (8, 16), None),
     "mx decode, narrow window": (64, 2048, 128, 8, 768, "f4e2m1", (8, 16), None),
     "bf16 decode, narrow window + live": (64, 2048, 128, 8, 768, "bf16", (8, 16), 40),
+    # 24 or more routes per expert: the decode front end (which quantises the hidden rows where the
+    # products take their scales token-major: e4m3, 128-channel gated rows) hands a window's routes over
+    # to the sort and the tiles
+    "fp8 decode, sort and tiles, window": (64, 640, 16, 8, 128, "f8e4m3", (4, 8), None),
+    "mx decode, sort and tiles, window": (64, 512, 16, 8, 256, "f4e2m1", (4, 8), None),
+    "bf16 decode, sort and tiles, window + live": (64, 512, 16, 8, 256, "bf16", (4, 8), 40),
+}
+
+#: Kernels (of the mangled names' form) that some of these cases are there to run.
+ROUTED_KERNELS = {
+    "fp8 5 tokens, 60 experts, 512 channels": ("split_scores_kernelILi1ELi8EE", "route_chunk_kernel"),
+    "mx 3 tokens, 1536 channels, window + live": ("split_front_kernelILi4ELi2EE",),
+    "bf16 7 tokens, 100 experts, top 10, 2560 channels": ("split_scores_kernelILi0ELi8EE", "route_chunk_kernel"),
+    "fp8 4 tokens, 60 experts, 512 channels": ("split_front_kernelILi4ELi1EE",),
+    "bf16 4 tokens, 100 experts, top 10, 2560 channels": ("split_front_kernelILi8ELi0EE",),
+    "mx 7 tokens, 160 experts": ("12front_kernel", "stream_mx_kernelILb0ELb1ELb1E"),
+    "fp8 decode, narrow window": ("local_front_kernel", "stream_fp8_kernelILb1ELb1ELi2ELb1E"),
+    "mx decode, narrow window": ("local_front_kernel", "stream_mx_kernelILb1ELb1ELb1E"),
+    "bf16 decode, narrow window + live": ("local_front_kernel", "wide_kernelILb1ELb1E"),
+    "fp8 decode, sort and tiles, window": ("12front_kernel", "tiled_fp8_kernel"),
+    "mx decode, sort and tiles, window": ("12front_kernel", "tiled_mx_kernel"),
+    "bf16 decode, sort and tiles, window + live": ("12front_kernel", "pair_kernel"),
 }
 
 
@@ -80,8 +105,13 @@ def test_layer_routing_options_against_the_oracle(device, case):
     layer = ops.MoeLayer(hidden, experts, top, intermediate, tokens, weight_dtype=wdtype)
     load = torch.full((experts,), 5, dtype=torch.int64, device=device)  # the load accumulates
     live_t = None if live is None else torch.tensor([live], dtype=torch.int32, device=device)
-    out = layer(x, router, up_dev, down_dev, router_bias=torch.from_numpy(bias).to(device), live_tokens=live_t,
-                mapping=torch.from_numpy(mapping).to(device), load=load, window=window, **args)
+    out = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=device)
+    options = dict(args, out=out, router_bias=torch.from_numpy(bias).to(device), live_tokens=live_t,
+                   mapping=torch.from_numpy(mapping).to(device), load=load, window=window)
+    if case in ROUTED_KERNELS:
+        names = kernels_of(lambda: layer(x, router, up_dev, down_dev, **options))
+        assert all(any(kernel in name for name in names) for kernel in ROUTED_KERNELS[case]), names
+    layer(x, router, up_dev, down_dev, **options)
     torch.cuda.synchronize()
     got = bf16_values(out)
     ids = layer.view("ids", torch.int32, (tokens, top)).cpu().numpy()

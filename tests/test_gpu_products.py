@@ -35,15 +35,15 @@ def routing(device, tokens, experts, top, skew, seed, emptied=None):
 
 CASES = {
     # name: tokens, hidden, experts, top, intermediate, skew
-    "30b decode (stream)": (64, 2048, 128, 8, 768, "uniform"),
-    "skewed decode (stream, one-row-block passes over tiles of many rows)": (128, 2048, 128, 8, 768, "zipf"),
-    "skewed decode (stream, two-row-block passes over tiles of many rows)": (256, 2048, 128, 8, 768, "zipf"),
+    "30b decode (wide)": (64, 2048, 128, 8, 768, "uniform"),
+    "skewed decode, tiles of many rows (wide)": (128, 2048, 128, 8, 768, "zipf"),
+    "skewed decode, tiles of up to four passes of rows (wide)": (256, 2048, 128, 8, 768, "zipf"),
     "reference gather shape, emptied expert": (512, 2048, 128, 8, 1536, "uniform"),
-    "skewed prefill (tiled)": (1024, 2048, 128, 8, 768, "zipf"),
+    "skewed prefill (pair)": (1024, 2048, 128, 8, 768, "zipf"),
     "tiny": (16, 256, 8, 2, 128, "uniform"),
     "235b decode one token": (1, 4096, 128, 8, 1536, "uniform"),
     "odd widths (tiled, 64-column slices)": (300, 320, 16, 4, 192, "uniform"),
-    "stream, hidden not a multiple of 256 (row-sliced FC1)": (16, 320, 16, 4, 192, "uniform"),
+    "hidden of whole 64-element steps only (tiled)": (16, 320, 16, 4, 192, "uniform"),
     "few experts of many rows (stream, two row blocks a pass)": (70, 384, 8, 2, 256, "zipf"),
     "FC2 of an odd number of 64 columns (stream, two row blocks a pass)": (72, 192, 8, 2, 256, "uniform"),
 }
@@ -65,6 +65,11 @@ def test_products_and_combine(device, case):
     rows = ops.permuted_rows(tokens, top, experts)
     gated = torch.full((rows, intermediate), float("nan"), dtype=torch.bfloat16, device=device)
     products = torch.full((rows, hidden), float("nan"), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: (ops.gather_gemm(x, up_gate, top, maps, rows, out=gated),
+                                ops.route_gemm(gated, down, maps, out=products)))
+    named = [word for word in ("wide", "stream", "tiled", "pair") if word in case]
+    claimed = names[1:] if case.startswith("FC2") else names
+    assert not named or all(named[0] + "_kernel" in name for name in claimed), names
     ops.gather_gemm(x, up_gate, top, maps, rows, out=gated)
     ops.route_gemm(gated, down, maps, out=products)
     combined = ops.moe_unpermute(products, maps[ops.EXPANDED_TO_PERMUTED][: tokens * top], weights)

@@ -1,6 +1,7 @@
 """The expert-major decode products where an expert has as many rows as a pass takes, one fewer, one
 more, several passes' worth, or more runs than there are workgroup columns for - and uneven K
-quarters - against the oracle's layer. A router bias sends every token to the same experts, so their
+quarters - against the oracle's layer. (Small e4m3 and MXFP4 layers take the split stream kernels; the
+wide ones are named in test_wide_kernels_of_many_rows.) A router bias sends every token to the same experts, so their
 row counts are the token count exactly."""
 
 import numpy as np
@@ -21,8 +22,8 @@ CASES = {
     "a pass and one": (33, 512, 64, 4, 256, None, None),
     "two passes and one, 20 and 6 lines of K": (65, 1280, 64, 4, 384, None, None),
     "some rows not live": (100, 512, 64, 4, 256, None, 70),
-    "fewer columns than passes": (300, 512, 128, 8, 256, (2, 3), None),
-    "fewer columns than passes, a run ends on a pass": (288, 512, 128, 8, 256, (0, 4), None),
+    "a window of three experts": (300, 512, 128, 8, 256, (2, 3), None),
+    "a window of four experts, a run ends on a pass": (288, 512, 128, 8, 256, (0, 4), None),
     "fewer routes than experts": (40, 512, 128, 2, 256, None, None),
 }
 
@@ -109,31 +110,48 @@ def test_which_walks_may_be_spread(device, case):
     assert ["Lb1ELb%dEE" % fc1 in pairs[0], "Lb0ELb%dEE" % fc2 in pairs[1]] == [True, True], names
 
 
-_FC1 = {"f8e4m3": "wide_fp8_kernelILb1ELi2ELi2ELb1EE", "f4e2m1": "wide_mx_kernelILb1ELi2ELi2ELb1EE"}
+_FP8, _MX = "wide_fp8_kernelILb", "wide_mx_kernelILb"
 WIDE = {
-    # name: weights, tokens, hidden, experts, top, intermediate, window, live, FC2's kernel. (At most 48
-    # runs past the first passes are shared out to columns of their own: eight experts of 300 rows have 72
-    # and take them 64 rows at a time, of 288 rows 64.)
-    "e4m3, window, FC2 of 4 lines": ("f8e4m3", 300, 1024, 128, 8, 512, (0, 16), None, "wide_fp8_kernelILb0ELi4ELi1ELb0EE"),
-    "e4m3, window, FC2 of 6 lines": ("f8e4m3", 288, 2048, 128, 8, 768, (0, 16), None, "wide_fp8_kernelILb0ELi2ELi2ELb0EE"),
-    "e4m3, window, some rows not live": ("f8e4m3", 200, 1024, 128, 8, 512, (4, 20), 150, "wide_fp8_kernelILb0ELi4ELi1ELb0EE"),
-    "mx, window, FC2 of 2 lines": ("f4e2m1", 300, 1024, 128, 8, 512, (0, 16), None, "wide_mx_kernelILb0ELi2ELi2ELb0EE"),
-    "mx, window, FC2 of 3 lines": ("f4e2m1", 288, 2048, 128, 8, 768, (0, 16), None, "wide_mx_kernelILb0ELi1ELi4ELb0EE"),
-    "mx, window, some rows not live": ("f4e2m1", 200, 1024, 128, 8, 768, (4, 20), 150, "wide_mx_kernelILb0ELi1ELi4ELb0EE"),
-    "bf16, window": ("bf16", 300, 512, 128, 8, 256, (0, 16), None, "wide_kernelILb0ELb1ELi2EE"),
+    # name: weights, tokens, hidden, experts, top, intermediate, window, live, FC1's and FC2's kernels. (At
+    # most 48 runs past the first passes are shared out to columns of their own, or as many as experts:
+    # eight experts of 300 rows have 72 and take them 64 rows at a time, of 288 rows 64.)
+    "e4m3, a pass and one": ("f8e4m3", 33, 1024, 64, 8, 512, None, None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+    "e4m3, two passes and one, some rows not live": (
+        "f8e4m3", 90, 2048, 64, 8, 768, None, 65, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi2ELi2ELb0EE"),
+    "e4m3, compact grid": (
+        "f8e4m3", 15, 4096, 128, 8, 512, None, None, _FP8 + "1ELi2ELi2ELb1EE", "stream_fp8_kernelILb0ELb0ELi1ELb1E"),
+    "e4m3, window, FC2 of 4 lines": (
+        "f8e4m3", 300, 1024, 128, 8, 512, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+    "e4m3, window, FC2 of 6 lines": (
+        "f8e4m3", 288, 2048, 128, 8, 768, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi2ELi2ELb0EE"),
+    "e4m3, window, some rows not live": (
+        "f8e4m3", 200, 1024, 128, 8, 512, (4, 20), 150, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+    "mx, a pass and one": ("f4e2m1", 33, 1024, 64, 8, 512, None, None, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi2ELi2ELb0EE"),
+    "mx, two passes and one, some rows not live": (
+        "f4e2m1", 90, 2048, 64, 8, 768, None, 65, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi1ELi4ELb0EE"),
+    "mx, compact grid": (
+        "f4e2m1", 12, 1024, 128, 8, 512, None, None, "stream_mx_kernelILb1ELb0ELb1ELi1ELb1EE", _MX + "0ELi2ELi2ELb0EE"),
+    "mx, window, FC2 of 2 lines": (
+        "f4e2m1", 300, 1024, 128, 8, 512, (0, 16), None, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi2ELi2ELb0EE"),
+    "mx, window, FC2 of 3 lines": (
+        "f4e2m1", 288, 2048, 128, 8, 768, (0, 16), None, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi1ELi4ELb0EE"),
+    "mx, window, some rows not live": (
+        "f4e2m1", 200, 1024, 128, 8, 768, (4, 20), 150, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi1ELi4ELb0EE"),
+    "bf16, window": ("bf16", 300, 512, 128, 8, 256, (0, 16), None, "wide_kernelILb1ELb1ELi2EE", "wide_kernelILb0ELb1ELi2EE"),
 }
 
 
 @pytest.mark.parametrize("case", list(WIDE))
-def test_wide_kernels_share_out_a_windows_rows(device, case):
-    """A window that holds the much-named experts takes the wide kernels, whose further columns share out
-    the rows past an expert's first pass."""
-    wdtype, tokens, hidden, experts, top, intermediate, window, live, fc2 = WIDE[case]
-    announce("wide kernels, window", case)
+def test_wide_kernels_of_many_rows(device, case):
+    """The wide kernels by name - also of a window that holds the much-named experts - where further
+    columns share out the rows past an expert's first pass."""
+    wdtype, tokens, hidden, experts, top, intermediate, window, live, fc1, fc2 = WIDE[case]
+    announce("wide kernels", case)
+    local = experts if window is None else window[1]
     x = normal_bf16((tokens, hidden), 101, device=device)
     router = normal_bf16((experts, hidden), 102, 0.02, device)
-    up_gate = normal_bf16((window[1], 2 * intermediate, hidden), 103, 0.02, device)
-    down = normal_bf16((window[1], hidden, intermediate), 104, 0.02, device)
+    up_gate = normal_bf16((local, 2 * intermediate, hidden), 103, 0.02, device)
+    down = normal_bf16((local, hidden, intermediate), 104, 0.02, device)
     bias = np.where(np.arange(experts) < top, 40.0, 0.0).astype(np.float32)
     bias_dev = torch.from_numpy(bias).to(device)
     live_t = None if live is None else torch.tensor([live], dtype=torch.int32, device=device)
@@ -145,7 +163,6 @@ def test_wide_kernels_share_out_a_windows_rows(device, case):
         layer(x, router, up_dev, down_dev, out=out, router_bias=bias_dev, live_tokens=live_t, window=window, **args)
 
     names = kernels_of(call)
-    fc1 = _FC1.get(wdtype, "wide_kernelILb1ELb1ELi2EE")
     assert any(fc1 in name for name in names) and any(fc2 in name for name in names), names
     call()
     torch.cuda.synchronize()
