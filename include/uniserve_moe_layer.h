@@ -60,8 +60,8 @@ UNISERVE_EXTERN_C int64_t uniserve_moe_layer_workspace(int64_t tokens, int64_t h
 
 /// Offsets (bytes from `workspace`) of the intermediate tensors, for callers that read them:
 /// scores, ids, weights, the seven sort maps, gated rows, products. At decode sizes (the fused
-/// front end, at most 4096 routes, fewer than 24 per local expert) the layer skips the sort, for
-/// every weight type: then expanded_to_permuted holds each route's own index (token * top + k)
+/// front end, at most 4096 routes, fewer than 24 per expert of the router - not of the window - and
+/// product widths the expert-major kernels take) the layer skips the sort, for every weight type: then expanded_to_permuted holds each route's own index (token * top + k)
 /// where the route is live and in the window and -1 elsewhere, the other six maps are not
 /// written, and gated rows and products (and the quantised gated rows and their scales) sit at
 /// those expanded positions.
@@ -128,8 +128,10 @@ UNISERVE_EXTERN_C int32_t uniserve_moe_layer_no_alloc(const struct uniserve_moe_
 /// The layer's launches in order. Which step launches what depends on the call's size:
 /// - decode sizes (at most 4096 routes over at most 512 local experts, a router of at most 1024
 ///   experts): ROUTER launches the front end - router scores and topk, plus the sort where the
-///   layer does not skip it, plus the hidden rows' e4m3 / MXFP8 quantisation for those weights, in one
-///   kernel or (without a sort, past 4 tokens) two - and TOPK, SORT and QUANTIZE_HIDDEN launch nothing;
+///   layer does not skip it, plus the hidden rows' e4m3 / MXFP8 quantisation for those weights - in
+///   two kernels without a sort for 5 to 31 tokens, for more than 256 and for more than 4 of 4096 channels
+///   or more (at most 128 experts, hidden a multiple of 128), else in one - and TOPK, SORT and
+///   QUANTIZE_HIDDEN launch nothing;
 /// - prefill sizes (at most 128 experts, hidden a multiple of 128): ROUTER launches router scores,
 ///   topk and the hidden rows' quantisation in one kernel, up to 4096 tokens in two (in a call that also
 ///   runs SORT, the sort's per-chunk counts too, so that SORT launches only its placement), TOPK launches
@@ -142,7 +144,8 @@ UNISERVE_EXTERN_C int32_t uniserve_moe_layer_no_alloc(const struct uniserve_moe_
 /// writes its rows already quantised (e4m3 at prefill sizes; MXFP4 with route-major scales; and, for
 /// both e4m3 and MXFP4, at decode sizes where the local experts with routes times intermediate / 64
 /// reach 512 - 30B at 64 tokens, not one token - with an intermediate size of whole 128-column
-/// groups for e4m3).
+/// groups for e4m3, or where a window of 16 experts or more has more than 64 tokens - MXFP4 under
+/// 4096 channels: of 32 or more, or more than 8 routes per expert).
 enum uniserve_moe_layer_step {
   UNISERVE_MOE_LAYER_ROUTER = 0,
   UNISERVE_MOE_LAYER_TOPK = 1,

@@ -718,8 +718,8 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
   const int64_t slices = gated ? e.out_width / 64 : e.out_width / 128;
   const dim3 grid(static_cast<uint32_t>(p.compact ? e.routes : e.local_experts), static_cast<uint32_t>(slices));
   if (wide_fits(p, e.routes) && (gated || e.routes > kWideFc2RowsPerExpert * e.experts)) {
-    // An expert with more rows than one pass takes leaves the rest to workgroups of their own (with
-    // one column per expert that may have any: nth_extra_run).
+    // An expert with more rows than one pass takes leaves the rest to workgroups of their own
+    // (extra_columns).
     const bool one_block = gated && e.routes <= kWideOneBlockRowsPerExpert * e.experts;
     p.extra_columns = extra_columns(e.routes, e.top, e.local_experts, p.compact != 0, one_block ? 16 : kWideRows);
     p.columns = static_cast<int32_t>(grid.x);

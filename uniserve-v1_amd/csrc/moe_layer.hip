@@ -350,7 +350,6 @@ int32_t run_layer(const uniserve_moe_layer_call *call, int32_t only, void *strea
                            expert_stream_fits(routes, call->experts, local_experts, call->hidden_size, call->intermediate, true) &&
                            expert_stream_fits(routes, call->experts, local_experts, call->intermediate, call->hidden_size, false) &&
                            (!mx || (call->hidden_size % 256 == 0 && call->intermediate % 256 == 0));
-    if (by_expert) v.route_scales = 0;  // (rows at expanded positions: no permuted rows to lay scales out by)
 
     // e4m3 and MXFP4 at those sizes: the front end also quantises the hidden rows (QUANTIZE_HIDDEN
     // then launches nothing).
