@@ -115,17 +115,21 @@ WIDE = {
     # name: weights, tokens, hidden, experts, top, intermediate, window, live, FC1's and FC2's kernels. (At
     # most 48 runs past the first passes are shared out to columns of their own, or as many as experts:
     # eight experts of 300 rows have 72 and take them 64 rows at a time, of 288 rows 64.)
-    "e4m3, a pass and one": ("f8e4m3", 33, 1024, 64, 8, 512, None, None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+    "e4m3, a pass and one": ("f8e4m3", 33, 1024, 64, 8, 1024, None, None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
     "e4m3, two passes and one, some rows not live": (
         "f8e4m3", 90, 2048, 64, 8, 768, None, 65, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi2ELi2ELb0EE"),
     "e4m3, compact grid": (
         "f8e4m3", 15, 4096, 128, 8, 512, None, None, _FP8 + "1ELi2ELi2ELb1EE", "stream_fp8_kernelILb0ELb0ELi1ELb1E"),
     "e4m3, window, FC2 of 4 lines": (
-        "f8e4m3", 300, 1024, 128, 8, 512, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+        "f8e4m3", 300, 1024, 128, 8, 512, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi2ELi2ELb0EE"),
+    "e4m3, window, FC2 of 4 lines, a width of an odd number of 128 columns": (
+        "f8e4m3", 100, 640, 128, 8, 512, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+    "e4m3, window, FC2 of 8 lines": (
+        "f8e4m3", 288, 512, 128, 8, 1024, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
     "e4m3, window, FC2 of 6 lines": (
         "f8e4m3", 288, 2048, 128, 8, 768, (0, 16), None, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi2ELi2ELb0EE"),
     "e4m3, window, some rows not live": (
-        "f8e4m3", 200, 1024, 128, 8, 512, (4, 20), 150, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
+        "f8e4m3", 200, 1024, 128, 8, 1024, (4, 20), 150, _FP8 + "1ELi2ELi2ELb1EE", _FP8 + "0ELi4ELi1ELb0EE"),
     "mx, a pass and one": ("f4e2m1", 33, 1024, 64, 8, 512, None, None, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi2ELi2ELb0EE"),
     "mx, two passes and one, some rows not live": (
         "f4e2m1", 90, 2048, 64, 8, 768, None, 65, _MX + "1ELi2ELi2ELb1EE", _MX + "0ELi1ELi4ELb0EE"),

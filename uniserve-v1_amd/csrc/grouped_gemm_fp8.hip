@@ -380,7 +380,7 @@ __global__ void __launch_bounds__(kWaves * kWave) stream_fp8_kernel(GroupedFp8Pa
 // (q + 1) L / kParts - 1), and the parts' sums meet in LDS, added in part order. A workgroup holds
 // kGroups runs of 128 weight rows. FC1: two parts, two runs - 128 gated columns, one whole scale group,
 // so with out_codes it also writes the gated rows as FC2's operand. FC2: four parts where they divide
-// the lines (235B: 12), else two parts and two runs (30B: 6 lines, three a part).
+// the lines into two or more each (235B: 12), else two parts and two runs (30B: 6 lines, three a part).
 //
 // Bound by HBM (30B T=128 FC1 64 us, 6.3 TB/s). Against the stream kernel (16 or 32 rows a pass, every
 // wavefront loading all the rows): 30B T=128 FC1 73 -> 64 us, FC2 39 -> 35; T=200 80 -> 69, 43.5 ->
@@ -866,6 +866,14 @@ bool split_fp8(const GroupedFp8Params &p, bool gated) {
 
 bool expert_stream_fp8_fc1_quantizes(const GroupedFp8Params &p) { return !split_fp8(p, true) && p.out_width % 128 == 0; }
 
+/// FC2 in four parts of K, not two: where they divide the lines into two or more each (four of one line
+/// spend their time on the exchange: 512 channels, 256 experts of top 8, hidden 2048, T=150 56 us against 46 with two
+/// parts and 45 on the stream kernel; with Zipf routing 45, 35 and 95), or where two do not fit the width.
+bool wide_fp8_four_parts(const GroupedFp8Params &p) {
+  const int64_t lines = p.K / 128;
+  return lines % 4 == 0 && (lines >= 8 || p.out_width % 256 != 0);
+}
+
 void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, hipStream_t stream) {
   GroupedFp8Params p = params;
   const int64_t local_experts = p.local_experts;
@@ -888,7 +896,7 @@ void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, hipStr
   if (wide_fp8_fits(p, gated)) {
     p.columns = static_cast<int32_t>(columns);
     p.extra_columns = extra_columns(p.routes, p.top, local_experts, p.compact != 0, kWideRows);
-    const bool four = p.K / 128 % 4 == 0;
+    const bool four = wide_fp8_four_parts(p);
     const int64_t runs = gated || four ? p.out_width / 128 : p.out_width / 256;
     const dim3 grid(static_cast<uint32_t>((p.columns + p.extra_columns) * runs));
     if (gated) hipLaunchKernelGGL((wide_fp8_kernel<true, 2, 2, true>), grid, dim3(kThreads), 0, stream, p);
