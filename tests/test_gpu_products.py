@@ -212,3 +212,37 @@ def test_expert_major_two_row_blocks(device, wdtype):
     np.testing.assert_array_equal(layer.view("ids", torch.int32, (tokens, top)).cpu().numpy(), want_ids)
     assert_bf16_bar(bf16_values(out), O.bf16_decode(want_bits).astype(np.float64), wdtype,
                     max_rel=2e-2 if wdtype == "bf16" else 4e-2)
+
+
+FEW_ROWS = {
+    # name: tokens, hidden, experts, top, FC1's kernel
+    "rows of 6 KB, three per expert": (96, 3072, 64, 2, "stream_kernelILb1ELi1ELb0EE"),
+    "rows of 6 KB, more": (97, 3072, 64, 2, "wide_kernelILb1ELb0ELi2EE"),
+    "rows of 4 KB": (6, 2048, 64, 2, "wide_kernelILb1ELb0ELi2EE"),
+}
+
+
+@pytest.mark.parametrize("case", list(FEW_ROWS))
+def test_few_rows_by_tiles(device, case):
+    """By the sort's tiles, FC1 of few rows per expert takes the wide kernel only at row strides of whole
+    4 KB."""
+    tokens, hidden, experts, top, kernel = FEW_ROWS[case]
+    announce("few rows by tiles", case)
+    intermediate = 1024
+    ids = torch.arange(tokens * top, device=device, dtype=torch.int32).reshape(tokens, top) % experts
+    maps = ops.moe_sort(ids, torch.rand((tokens, top), device=device), experts)
+    rows = ops.permuted_rows(tokens, top, experts)
+    x = normal_bf16((tokens, hidden), 21, device=device)
+    up_gate = normal_bf16((experts, 2 * intermediate, hidden), 22, 0.02, device)
+    gated = torch.zeros((rows, intermediate), dtype=torch.bfloat16, device=device)
+    names = kernels_of(lambda: ops.gather_gemm(x, up_gate, top, maps, rows, out=gated))
+    assert kernel in names[-1], names
+    ops.gather_gemm(x, up_gate, top, maps, rows, out=gated)
+    torch.cuda.synchronize()
+    route = maps[ops.EXPANDED_TO_PERMUTED][: tokens * top].long()
+    want = torch.empty((tokens * top, intermediate), device=device)
+    for e in range(experts):
+        named = torch.nonzero(ids.reshape(-1) == e).reshape(-1)
+        both = x[named // top].float() @ up_gate[e].float().t()
+        want[named] = torch.nn.functional.silu(both[:, intermediate:]) * both[:, :intermediate]
+    assert_bf16_bar(bf16_values(gated[route]), want.cpu().numpy().astype(np.float64), case, max_rel=2e-2)

@@ -18,11 +18,10 @@
 //    every touched expert's matrix is read from HBM and little else matters. A workgroup owns 128
 //    weight rows and 32 activation rows, its wavefronts a quarter of K each.
 //
-//  * `stream` (FC2 of the smallest batches, FC2 widths of an odd number of 64 columns, few experts, and K
-//    below 256): a 128-row slice of the expert's weight rows per workgroup, each wavefront streaming its
-//    own 32 rows over all of K. The weight lines are
-//    regrouped into the MFMA operand layout through LDS, the activation rows come from L2. The weight
-//    rows are MFMA operand A and the activation rows operand B (16x16x32 bf16), so each lane ends
+//  * `stream` (FC2 and, by tiles, FC1 of the smallest batches, FC2 widths of an odd number of 64 columns,
+//    few experts, and K below 256): a 128-row slice of the expert's weight rows per workgroup, each
+//    wavefront streaming its own 32 rows over all of K. The weight lines are regrouped into the MFMA operand
+//    layout through LDS, the activation rows come from L2. The weight rows are MFMA operand A and the activation rows operand B (16x16x32 bf16), so each lane ends
 //    holding four consecutive output columns of one row - an 8-byte store - and the SiLU pair (up
 //    column n, gate column n) meets in one lane.
 //
@@ -630,11 +629,11 @@ __global__ void __launch_bounds__(kThreads) tiled_kernel(GroupedParams p) {
 /// The stream and wide kernels serve batches whose experts average fewer rows than this.
 constexpr int64_t kStreamRowsPerExpert = 24;
 
-/// FC2 by expert with at most this many rows per expert on average stays on the stream kernel,
-/// whose workgroups need no exchange of partial sums (30B: T=5 21.1 us against 23.4 on the wide
+/// FC2, and by the sort's tiles FC1 of most widths, with at most this many rows per expert on average stay
+/// on the stream kernel, whose workgroups need no exchange of partial sums (30B FC2: T=5 21.1 us against 23.4 on the wide
 /// kernel, T=40 58.2 against 59.5, T=64 61.8 against 61.8 - with Zipf routing, where some experts have more than 16 rows, 86
 /// against 50 - and T=128 70 against 65).
-constexpr int64_t kWideFc2RowsPerExpert = 3;
+constexpr int64_t kWideFewRowsPerExpert = 3;
 
 /// FC1 by expert with at most this many rows per expert on average: 16 rows a pass, whose fewer
 /// registers leave three waves per SIMD (30B: T=32 104 us against 107, T=64 117.5 against 118.3, with
@@ -653,7 +652,10 @@ bool wide_fits(const GroupedParams &p, int64_t act_rows) {
 template <bool kGated>
 void launch_grouped(const GroupedParams &p, int64_t max_tiles, int64_t act_rows, int64_t routes, int64_t experts, hipStream_t s) {
   const bool stream_path = routes < kStreamRowsPerExpert * experts && p.K % 128 == 0;
-  const bool few_rows = !kGated && routes <= kWideFc2RowsPerExpert * experts;
+  // (FC1 rows of whole 4 KB gain by the wide kernel's walk at any count: 30B T=16 86 -> 81 us, T=64 144 -> 124. Others
+  // lose by it below a few rows per expert - K = 3072, 64 experts of top 6, T=6 79.5 -> 89.5, K = 1536, 60 of top 4,
+  // T=32 43 -> 48 - and above are slower near-uniform, T=64 46 -> 51, and much faster with Zipf routing, 57 -> 37.)
+  const bool few_rows = routes <= kWideFewRowsPerExpert * experts && (!kGated || p.K * 2 % 4096 != 0);
 
   if (!stream_path && (pair_fits<pair::Bf16>(kGated, p.K, p.out_width, 0) || prefill_fits<prefill::Bf16, kGated>(p.K, p.out_width))) {
     PrefillParams q{};
@@ -677,7 +679,7 @@ void launch_grouped(const GroupedParams &p, int64_t max_tiles, int64_t act_rows,
   const dim3 grid(static_cast<uint32_t>(max_tiles), static_cast<uint32_t>(slices));
   // Below two wide workgroups per three CUs the stream kernel, whose workgroups end without an exchange
   // of partial sums (30B T=1: FC1 14.3 us against 16.6; 235B T=1, 192 workgroups: 35.8 against 34.2).
-  if (stream_path && max_tiles * slices >= kWideWorkgroups && (kGated || (!few_rows && p.out_width % 128 == 0)) &&
+  if (stream_path && max_tiles * slices >= kWideWorkgroups && !few_rows && (kGated || p.out_width % 128 == 0) &&
       wide_fits(p, act_rows))
     hipLaunchKernelGGL((wide_kernel<kGated, false>), grid, dim3(kThreads), 0, s, p);
   else if (stream_path && routes <= kOnePassRowsPerExpert * experts)
@@ -717,7 +719,7 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
   p.compact = e.routes < e.local_experts ? 1 : 0;
   const int64_t slices = gated ? e.out_width / 64 : e.out_width / 128;
   const dim3 grid(static_cast<uint32_t>(p.compact ? e.routes : e.local_experts), static_cast<uint32_t>(slices));
-  if (wide_fits(p, e.routes) && (gated || e.routes > kWideFc2RowsPerExpert * e.experts)) {
+  if (wide_fits(p, e.routes) && (gated || e.routes > kWideFewRowsPerExpert * e.experts)) {
     // An expert with more rows than one pass takes leaves the rest to workgroups of their own
     // (extra_columns).
     const bool one_block = gated && e.routes <= kWideOneBlockRowsPerExpert * e.experts;
