@@ -63,6 +63,8 @@ ROUTED = {
     "fp8 decode, narrow window": (64, 2048, 128, 8, 768, "f8e4m3", (8, 16), None),
     "mx decode, narrow window": (64, 2048, 128, 8, 768, "f4e2m1", (8, 16), None),
     "bf16 decode, narrow window + live": (64, 2048, 128, 8, 768, "bf16", (8, 16), 40),
+    "bf16 40 tokens, narrow window": (40, 2048, 128, 8, 768, "bf16", (8, 16), None),
+    "fp8 24 tokens, narrow window, wide rows": (24, 4096, 128, 8, 256, "f8e4m3", (8, 16), None),
     # 24 or more routes per expert: the decode front end (which quantises the hidden rows where the
     # products take their scales token-major: e4m3, 128-channel gated rows) hands a window's routes over
     # to the sort and the tiles
@@ -82,6 +84,8 @@ ROUTED_KERNELS = {
     "fp8 decode, narrow window": ("local_front_kernel", "stream_fp8_kernelILb1ELb1ELi2ELb1E"),
     "mx decode, narrow window": ("local_front_kernel", "stream_mx_kernelILb1ELb1ELb1E"),
     "bf16 decode, narrow window + live": ("local_front_kernel", "wide_kernelILb1ELb1E"),
+    "bf16 40 tokens, narrow window": ("local_front_kernel", "stream_kernelILb0ELi1ELb1EE"),
+    "fp8 24 tokens, narrow window, wide rows": ("split_scores_kernelILi1ELi8EE", "stream_fp8_kernelILb0ELb0ELi1ELb1E"),
     "fp8 decode, sort and tiles, window": ("12front_kernel", "tiled_fp8_kernel"),
     "mx decode, sort and tiles, window": ("12front_kernel", "tiled_mx_kernel"),
     "bf16 decode, sort and tiles, window + live": ("12front_kernel", "pair_kernel"),

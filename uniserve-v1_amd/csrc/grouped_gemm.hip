@@ -21,9 +21,9 @@
 //  * `stream` (FC2 and, by tiles, FC1 of the smallest batches, FC2 widths of an odd number of 64 columns,
 //    few experts, and K below 256): a 128-row slice of the expert's weight rows per workgroup, each
 //    wavefront streaming its own 32 rows over all of K. The weight lines are regrouped into the MFMA operand
-//    layout through LDS, the activation rows come from L2. The weight rows are MFMA operand A and the activation rows operand B (16x16x32 bf16), so each lane ends
-//    holding four consecutive output columns of one row - an 8-byte store - and the SiLU pair (up
-//    column n, gate column n) meets in one lane.
+//    layout through LDS, the activation rows come from L2. The weight rows are MFMA operand A and the
+//    activation rows operand B (16x16x32 bf16), so each lane ends holding four consecutive output columns
+//    of one row - an 8-byte store - and the SiLU pair (up column n, gate column n) meets in one lane.
 //
 //  * `prefill` (grouped_prefill.hpp; hundreds of rows per expert): 128 x 512 tiles of 8
 //    wavefronts, both operands DMA'd into LDS, for the shapes it serves.
@@ -732,7 +732,7 @@ void launch_expert_stream(const ExpertStream &e, bool gated, hipStream_t stream)
     else hipLaunchKernelGGL((wide_kernel<false, true>), wide_grid, dim3(kThreads), 0, stream, p);
     return;
   }
-  const bool one_pass = e.routes <= kOnePassRowsPerExpert * e.local_experts;
+  const bool one_pass = e.routes <= kOnePassRowsPerExpert * e.experts;
   if (gated && one_pass) hipLaunchKernelGGL((stream_kernel<true, 1, true>), grid, dim3(kThreads), 0, stream, p);
   else if (gated) hipLaunchKernelGGL((stream_kernel<true, 2, true>), grid, dim3(kThreads), 0, stream, p);
   else if (one_pass) hipLaunchKernelGGL((stream_kernel<false, 1, true>), grid, dim3(kThreads), 0, stream, p);

@@ -912,7 +912,8 @@ void launch_expert_stream_fp8(const GroupedFp8Params &params, bool gated, hipStr
   }
   const dim3 grid(static_cast<uint32_t>(columns), static_cast<uint32_t>(slices));
   if (gated) hipLaunchKernelGGL((stream_fp8_kernel<true, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
-  else if (one_pass) hipLaunchKernelGGL((stream_fp8_kernel<false, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
+  else if (p.routes <= kOnePassRowsPerExpert * p.experts)  // (an expert's rows, whatever the window)
+    hipLaunchKernelGGL((stream_fp8_kernel<false, false, 1, true>), grid, dim3(kThreads), 0, stream, p);
   else hipLaunchKernelGGL((stream_fp8_kernel<false, false, 2, true>), grid, dim3(kThreads), 0, stream, p);
 }
 
