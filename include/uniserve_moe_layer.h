@@ -145,7 +145,7 @@ UNISERVE_EXTERN_C int32_t uniserve_moe_layer_no_alloc(const struct uniserve_moe_
 /// both e4m3 and MXFP4, at decode sizes where the local experts with routes times intermediate / 64
 /// reach 512 - 30B at 64 tokens, not one token - with an intermediate size of whole 128-column
 /// groups for e4m3, or where a window of 16 experts or more has more than 64 tokens - MXFP4 under
-/// 4096 channels: of 32 or more, or more than 8 routes per expert).
+/// 4096 channels: of 32 or more, or more than 12 routes per expert).
 enum uniserve_moe_layer_step {
   UNISERVE_MOE_LAYER_ROUTER = 0,
   UNISERVE_MOE_LAYER_TOPK = 1,

@@ -1191,14 +1191,14 @@ bool wide_mx_fits(const MxParams &p, bool gated, int64_t experts) {
 /// wide passes of rows, which a split workgroup takes 16 at a time and the wide kernel shares out. Layer,
 /// sixteen of 128 experts from the first, Zipf, split -> wide: 30B T=200 137 -> 62 us, T=383 230 -> 92, 235B
 /// T=100 177 -> 91, T=383 607 -> 215; near-uniform 30B T=200 42 -> 43, T=383 54 -> 50, 235B T=100 63 -> 57. Fewer
-/// than 32 experts with rows of less than 4096 channels only above eight per expert (30B T=100 near-uniform
-/// 37.5 -> 40; 32 experts 47 -> 41), and not eight experts, whose columns are too few (T=200 38 -> 41).
+/// than 32 experts with rows of less than 4096 channels only above twelve per expert (30B T=130 near-uniform
+/// 37 -> 41; 32 experts T=100 47 -> 41), and not eight experts, whose columns are too few (T=200 38 -> 41).
 bool split_mx(const MxParams &p, bool gated, int64_t experts) {
   // Workgroups with routes: at most one per route.
   const int64_t served = p.routes < p.local_experts ? p.routes : p.local_experts;
   if (served * (p.out_width / (gated ? 64 : 128)) >= kSplitBelow) return false;
   const bool shared_out = p.local_experts >= kWideExperts && p.routes > 2 * kWideRows * p.top &&
-                          (p.K >= 4096 || p.local_experts >= 2 * kWideExperts || p.routes > 8 * experts);
+                          (p.K >= 4096 || p.local_experts >= 2 * kWideExperts || p.routes > 12 * experts);
   return !(shared_out && wide_mx_fits(p, gated, experts));
 }
 
